@@ -447,7 +447,8 @@ static void launch_recon(const Ctx &x, const float *vp, const float *u_prev, con
 {
     TimedScope ts(K_RECON);
     const Geo &g = x.g;
-    if (x.zm) {
+    const int64_t cells = int64_t(bx.x1 - bx.x0) * (bx.y1 - bx.y0) * (bx.z1 - bx.z0) * g.B;
+    if (x.zm && (x.zm_forced || cells >= kZmMinRecon3)) {
         launch_recon_zm(x, vp, u_prev, u_now, u_next, adj, grad, bx.x0, bx.x1, bx.y0, bx.y1, bx.z0, bx.z1);
         return;
     }
@@ -944,14 +945,15 @@ Ctx make_ctx(const swp_problem &p)
     x.tz = tuning(SWP_TUNE_TZ3, "SWP_TZ3", 64);
     // Kernel family, as in 2-D: the z-marching kernels from kZmMinCells3
     // shot-cells (B x nz x ny x nx on the runtime grid) up, one thread per
-    // cell below, where the few long z-march segments of a small launch are
-    // latency-bound (40 x 36 x 44, one shot: 672 against 37 us per step of
-    // forward + backward; the two meet near 41M shot-cells).
-    // SWP_KERNELS=percell / zmarch forces a family.
+    // cell below, where a launch holds too few z segments.
+    // SWP_KERNELS=percell / zmarch forces a family (zmarch_big: with the
+    // roundings of kBigCells3 shot-cells and up).
     const char *kern = std::getenv("SWP_KERNELS");
     const std::string ks = kern ? kern : "";
     const int64_t cells = int64_t(x.g.B) * x.g.nz * x.g.ny * x.g.nx;
-    x.zm = zm_supported(x.g, x.tz) && ks != "percell" && (ks == "zmarch" || cells >= kZmMinCells3);
+    x.big = cells >= kBigCells3 || ks == "zmarch_big";
+    x.zm_forced = ks == "zmarch" || ks == "zmarch_big";
+    x.zm = zm_supported(x.g, x.tz) && ks != "percell" && (ks == "zmarch" || ks == "zmarch_big" || cells >= kZmMinCells3);
     // SWP_SHELL3=percell runs the CPML shell with the per-cell kernels over
     // six slabs instead of the region-specialised z-marching kernels.
     const char *sh = std::getenv("SWP_SHELL3");

@@ -6,11 +6,25 @@
 namespace swp {
 namespace a3d {
 
+// Smallest launch (shots x runtime-grid cells) that runs on the z-marching
+// kernels by default; smaller ones run one thread per cell.  Measured per step
+// of forward + adjoint + reconstruction, order 8 (per-cell / z-march): 3.1M
+// shot-cells 164 / 164 us, 6.2M 394 / 310, 9.7M 571 / 425, 12.5M 686 / 452.
+constexpr int64_t kZmMinCells3 = int64_t(4) << 20;
+// From here up the forward step adds the last axes' second derivatives to the
+// CPML sum in one rounding each; below, every term is rounded first, as the
+// per-cell kernels do, so that a record there does not depend on the family.
+// (The records of either range keep the bits they had before the families'
+// border moved down from this size; the times are equal.)
+constexpr int64_t kBigCells3 = int64_t(32) << 20;
+// Smallest reconstruction box (shots x cells) on its z-marching kernel: the
+// box holds far fewer cells than the grid, and its kernel walks whole z
+// segments (1.4M cells 47 us against 16 us per-cell; from 2M to 8M the step
+// times are within 1.5%).
+constexpr int64_t kZmMinRecon3 = int64_t(4) << 20;
+
 // Orders 2..8, and a z segment of tz planes plus its 2M + 1 halo and prefetch
 // planes addressable with 32-bit byte offsets (tz is clamped to fit).
-// Smallest launch (shots x runtime-grid cells) that runs on the z-marching
-// kernels by default; smaller ones run one thread per cell.
-constexpr int64_t kZmMinCells3 = int64_t(32) << 20;
 
 bool zm_supported(const Geo &g, int &tz);
 // The slabs of the computed box around the lean interior [lo + M + 1,

@@ -13,11 +13,17 @@
 //
 // The computed box is cut into a lean interior -- [lo + M + 1, hi - M - 1)
 // per axis: no forward CPML term, no strip cell, no adjoint CPML term (the
-// adjoint's pure region) -- run by the *_int kernels, and six slabs around
-// it run by the *_shell kernels, which evaluate each cell's CPML bands.
-// Block indices are remapped so that each XCD (workgroups go round-robin
-// over the eight) takes a contiguous run of tiles, whose halos then meet in
-// the same L2.
+// adjoint's pure region) -- and the margins around it, grouped by the axes
+// whose CPML margin they lie in (eight types, the interior included).  One
+// launch per step runs every type: a workgroup looks its tile up in the plan
+// and takes the code compiled for its type.  The types were a launch each
+// before; on a volume of a few million cells each of those sixteen launches a
+// step (forward and adjoint) ran for its own 30 to 60 us however few cells it
+// held (97 x 110 x 131, order 8, one shot: 0.77 ms a step, per-cell kernels
+// 0.56 ms, one launch 0.37 ms); at 256 x 512 x 512 the two are equal.
+// Workgroup numbers are remapped so that each XCD (workgroups go round-robin
+// over the eight) takes a contiguous run of each type's tiles, whose halos
+// then meet in the same L2.
 //
 // The arithmetic is that of the per-cell kernels (acoustic3d.hip), which
 // follow the reference's expression trees (csrc/cuda/equations/acoustic3d/
@@ -63,15 +69,17 @@ __device__ __forceinline__ void static_for(F &&f)
     }
 }
 
-// One shot's field seen from plane zbase on through a raw buffer resource
-// (base and extent in SGPRs).  A load or store takes the lane's in-plane byte
-// offset (a loop-invariant VGPR) and the plane's byte offset (an SGPR), so a
-// plane step costs one scalar multiply instead of a 64-bit address per lane.
-// Accesses past the field's end read 0 and write nothing.  The caller keeps
-// (planes used) * sxy * 4 below 2^32.
-struct Fld {
+// One shot's field seen from plane zbase on.  An access takes the lane's
+// in-plane byte offset (a loop-invariant VGPR) and the plane's byte offset (an
+// SGPR); the caller keeps (planes used) * sxy * 4 below 2^32 and every row,
+// column and plane in the grid.  Two forms of the same access:
+// Buf, a raw buffer resource (four SGPRs, base and extent; past the field's
+// end loads read 0 and stores write nothing), where a plane step costs no
+// vector instruction -- the forward step and the reconstruction, which have
+// SGPRs for it (record of 128 x 256 x 256, order 8: 35.7 ms, with Ptr 36.9);
+struct Buf {
     __amdgpu_buffer_rsrc_t r;
-    __device__ __forceinline__ Fld(const float *field, int64_t base_cell, int64_t end_cell)
+    __device__ __forceinline__ Buf(const float *field, int64_t base_cell, int64_t end_cell)
     {
         const int64_t bytes = (end_cell - base_cell) * 4;
         r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(field + base_cell), short(0),
@@ -86,42 +94,83 @@ struct Fld {
     {
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, voff, soff, 0);
     }
-    // Streaming forms (non-temporal cache policy) for data no other lane of
-    // the step reads again, so it does not push the shared halo planes out of L2.
-    __device__ __forceinline__ float ld_nt(uint32_t voff, uint32_t soff) const
+};
+// Ptr, a base pointer (two SGPRs) and one 32-bit add a row and plane that all
+// fields share -- the adjoint, whose nineteen fields as resources spilled up
+// to 360 SGPRs to VGPR lanes (gradient of 256 x 512 x 512, two shots, 100
+// steps: 556 ms, with Buf 561).
+struct Ptr {
+    char *p;
+    __device__ __forceinline__ Ptr(const float *field, int64_t base_cell)
+        : p(reinterpret_cast<char *>(const_cast<float *>(field) + base_cell))
     {
-        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
     }
-    __device__ __forceinline__ void st_nt(float v, uint32_t voff, uint32_t soff) const
+    __device__ __forceinline__ float ld(uint32_t voff, uint32_t soff) const
     {
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, voff, soff, 0);
+        return *reinterpret_cast<const float *>(p + uint32_t(voff + soff));
+    }
+    __device__ __forceinline__ void st(float v, uint32_t voff, uint32_t soff) const
+    {
+        *reinterpret_cast<float *>(p + uint32_t(voff + soff)) = v;
     }
 };
 
-// This block's shot, tile origin and z segment; false for a block with no
-// work (never happens for a well-formed set).
-template <int TY>
-__device__ __forceinline__ bool zcoords(const ZSet &s, int &b, int &k, int &xo, int &yo, int &zb, int &ze)
+// One workgroup's tile: its rectangle, shot, tile origin and z segment.
+struct ZTile {
+    ZRect r;
+    int b, xo, yo, zb, ze;
+};
+
+// Tile t of one shot's tiles over n rectangles (TY rows each); false past the last.
+__device__ __forceinline__ bool ztile(const ZRect *rs, int n, int TY, int t, ZTile &out)
 {
-    const int total = int(gridDim.x);
-    const int f = int(xcd_local_id(blockIdx.x, unsigned(total)));
-    b = f / s.per_shot;
-    int t = f % s.per_shot;
-    for (k = 0; k < s.n; ++k) {
-        const ZRect &R = s.r[k];
+    for (int k = 0; k < n; ++k) {
+        const ZRect &R = rs[k];
         if (t < R.nblk) {
             const int tx = t % R.ntx;
             const int ty = (t / R.ntx) % R.nty;
             const int sg = t / (R.ntx * R.nty);
-            xo = R.xs + 64 * tx;
-            yo = R.y0 + TY * ty;
-            zb = R.z0 + sg * R.tz;
-            ze = min(zb + R.tz, R.z1);
+            out.r = R;
+            out.xo = R.xs + 64 * tx;
+            out.yo = R.y0 + TY * ty;
+            out.zb = R.z0 + sg * R.tz;
+            out.ze = min(out.zb + R.tz, R.z1);
             return true;
         }
         t -= R.nblk;
     }
     return false;
+}
+
+// The tile of a launch over one set, in the XCD-local order.
+template <int TY>
+__device__ __forceinline__ bool zcoords(const ZSet &s, ZTile &out)
+{
+    const int f = int(xcd_local_id(blockIdx.x, gridDim.x));
+    out.b = f / s.per_shot;
+    return ztile(s.r, s.n, TY, f % s.per_shot, out);
+}
+
+// The regions of a step in one launch.  Entry k is a region type (bit 0 BX,
+// bit 1 BY, bit 2 BZ) with its rectangles r[r0[k] .. r0[k + 1]) and the
+// workgroups [first[k], first[k + 1]): a multiple of eight, the last few
+// idle, so that every type is spread over the XCDs and numbered XCD-locally
+// by itself.
+struct ZPlan {
+    ZRect r[27];
+    int r0[9], first[9], type[8], per_shot[8], ty[8];
+    int n;
+};
+
+__device__ __forceinline__ bool zplan_tile(const ZPlan &zp, int B, int &type, ZTile &out)
+{
+    const int f = int(blockIdx.x);
+    int k = 0;
+    while (k + 1 < zp.n && f >= zp.first[k + 1]) ++k;
+    const int t = int(xcd_local_id(unsigned(f - zp.first[k]), unsigned(zp.first[k + 1] - zp.first[k])));
+    type = zp.type[k];
+    out.b = t / zp.per_shot[k];
+    return out.b < B && ztile(zp.r + zp.r0[k], zp.r0[k + 1] - zp.r0[k], zp.ty[k], t % zp.per_shot[k], out);
 }
 
 // ---------------------------------------------------------------- plane I/O
@@ -230,21 +279,41 @@ struct XHalo {
 // (when the neighbouring tiles fetch that plane as their own head, so the
 // shared lines are still in L2) and waits in an (M + 1)-deep queue until the
 // plane is staged in LDS; halo slot p mod (M + 1) holds plane zb + p.
-template <int M, int RY, bool BX, bool BY, bool BZ, int NW>
-__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) fwd3_kernel(Geo g, Coef c, Prof pr, StepFields f, float *__restrict__ u_this,
-                                                   float *__restrict__ strip, ZSet zs)
+// One axis' CPML update of a cell: its term of w_sum, and psi and zeta after
+// the step.  Which products are fused is written out, not left to the
+// compiler, so that a record's bits depend neither on the code around the sum
+// nor, below kBigCells3, on the kernel family (there every plain second
+// derivative enters the sum rounded and b du is the fused product of psi, as
+// in the per-cell kernel; see BIG in fwd3_tile for the sizes above).
+template <bool FUSE_APSI>
+__device__ __forceinline__ float cpml_axis(float L, float a, float b, float db, float da, float du, float dpsi,
+                                           float psi0, float zeta0, float &psi1, float &zeta1)
+{
+    const float tmp = fd::fused(da, psi0, fd::fused(dpsi, a, fd::fused(L, 1.0f + b, fd::rounded(db * du))));
+    const float az = fd::rounded(a * zeta0);
+    psi1 = FUSE_APSI ? fd::fused(a, psi0, fd::rounded(b * du)) : fd::fused(du, b, fd::rounded(a * psi0));
+    zeta1 = fd::fused(b, tmp, az);
+    return fd::rounded(fd::fused(1.0f + b, tmp, az));
+}
+
+template <int M, int RY, bool BX, bool BY, int NW>
+constexpr int fwd_plane() { return (1 + (BX ? 1 : 0) + (BY ? 1 : 0)) * (NW * RY + 2 * M) * (64 + 2 * M); }
+
+template <int M, int RY, bool BX, bool BY, bool BZ, int NW, bool BIG>
+__device__ __forceinline__ void fwd3_tile(const Geo &g, const Coef &c, const Prof &pr, const StepFields &f,
+                                          float *__restrict__ u_this, float *__restrict__ strip, const ZTile &tile,
+                                          float *lds_mem)
 {
     constexpr bool SHELL = BX || BY || BZ;
+    constexpr bool TAIL_Y = BIG && !BY && !BZ, TAIL_Z = BIG && !BZ;
     constexpr int TY = NW * RY;
     using PM = PlaneMap<M, TY, NW>;
     constexpr int LW = PM::LW, PS = PM::LH * PM::LW, YH = PM::YH;
-    constexpr int NPL = 1 + (BX ? 1 : 0) + (BY ? 1 : 0);
     constexpr int SX = 1, SY = BX ? 2 : 1;   // plane slots of psi_x, psi_y
     constexpr int R = 2 * M + 2, H = M + 1;
-    __shared__ float lds[2][NPL * PS];
-    int b, k, xo, yo, zb, ze;
-    if (!zcoords<TY>(zs, b, k, xo, yo, zb, ze)) return;
-    const ZRect Rc = zs.r[k];
+    float *const lds[2] = {lds_mem, lds_mem + fwd_plane<M, RY, BX, BY, NW>()};
+    const int b = tile.b, xo = tile.xo, yo = tile.yo, zb = tile.zb, ze = tile.ze;
+    const ZRect &Rc = tile.r;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int nx = g.nx, ny = g.ny;
     const int64_t sxy = g.sxy;
@@ -259,10 +328,10 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4)
     const int64_t mb = int64_t(b) * g.mstride + int64_t(zbase) * sxy, me = int64_t(b) * g.mstride + g.n;
     const uint32_t sxy4 = uint32_t(sxy) * 4u;
     auto pl = [&](int z) { return uint32_t(z - zbase) * sxy4; };
-    const Fld un(f.u_now, fb, fe), up(f.u_prev, fb, fe), unx(f.u_next, fb, fe), vp(f.vp, mb, me);
-    const Fld psx(f.psi[0], fb, fe), psy(f.psi[1], fb, fe), psz(f.psi[2], fb, fe);
-    const Fld pnx(f.psin[0], fb, fe), pny(f.psin[1], fb, fe), pnz(f.psin[2], fb, fe);
-    const Fld zex(f.zeta[0], fb, fe), zey(f.zeta[1], fb, fe), zez(f.zeta[2], fb, fe);
+    const Buf un(f.u_now, fb, fe), up(f.u_prev, fb, fe), unx(f.u_next, fb, fe), vp(f.vp, mb, me);
+    const Buf psx(f.psi[0], fb, fe), psy(f.psi[1], fb, fe), psz(f.psi[2], fb, fe);
+    const Buf pnx(f.psin[0], fb, fe), pny(f.psin[1], fb, fe), pnz(f.psin[2], fb, fe);
+    const Buf zex(f.zeta[0], fb, fe), zey(f.zeta[1], fb, fe), zez(f.zeta[2], fb, fe);
 
     uint32_t col[RY], yhc[YH];   // in-plane byte offsets
 #pragma unroll
@@ -311,17 +380,17 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4)
         const uint32_t so = pl(zn);
 #pragma unroll
         for (int r = 0; r < RY; ++r) {
-            nup[r] = up.ld_nt(col[r], so);
-            nv[r] = vp.ld_nt(col[r], so);
+            nup[r] = up.ld(col[r], so);
+            nv[r] = vp.ld(col[r], so);
             if constexpr (BX) {
                 npx[r] = psx.ld(col[r], so);
-                nzx[r] = zex.ld_nt(col[r], so);
+                nzx[r] = zex.ld(col[r], so);
             }
             if constexpr (BY) {
                 npy[r] = psy.ld(col[r], so);
-                nzy[r] = zey.ld_nt(col[r], so);
+                nzy[r] = zey.ld(col[r], so);
             }
-            if constexpr (BZ) nzz[r] = zez.ld_nt(col[r], so);
+            if constexpr (BZ) nzz[r] = zez.ld(col[r], so);
         }
         if constexpr (BX)
             if (xh.lds >= 0) npxh = psx.ld(xh.off, so);
@@ -416,29 +485,29 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4)
             const float *Rw = P + row;
             const float u0 = q[r][C];
             auto qz = [&](int t) { return q[r][(C + t + R) % R]; };
-            const float lx = lap_taps<M>(c, [&](int t) { return Rw[t]; }, g.inv_dx2);
-            const float ly = lap_taps<M>(c, [&](int t) { return Rw[t * LW]; }, g.inv_dy2);
-            const float lz = lap_taps<M>(c, qz, g.inv_dz2);
+            const float acc_x = lap_taps<M>(c, [&](int t) { return Rw[t]; }, 1.0f), lx = fd::rounded(fd::scaled(acc_x, g.inv_dx2));
+            const float acc_y = lap_taps<M>(c, [&](int t) { return Rw[t * LW]; }, 1.0f), ly = fd::rounded(fd::scaled(acc_y, g.inv_dy2));
+            const float acc_z = lap_taps<M>(c, qz, 1.0f), lz = fd::rounded(fd::scaled(acc_z, g.inv_dz2));
             float w_sum;
             if constexpr (!SHELL) {
-                w_sum = lx + ly + lz;
+                w_sum = BIG ? fd::plus_scaled<true>(fd::plus_scaled<true>(ly, acc_x, g.inv_dx2), acc_z, g.inv_dz2) : lx + ly + lz;
             } else {
                 if (strip) save_strips(g, strip + int64_t(b) * g.ns, L.x, L.y[r], z, u0);
                 const bool bandx = BX && inbx, bandy = BY && inby[r], bandz = BZ && inbz;
                 if (!bandx && !bandy && !bandz) {
-                    w_sum = lx + ly + lz;
+                    w_sum = fd::plus_scaled<TAIL_Z>(fd::plus_scaled<TAIL_Y>(lx, acc_y, g.inv_dy2), acc_z, g.inv_dz2);
                 } else {
                     w_sum = 0.f;
+                    float psi1, z1v;
                     if (bandx) {
                         const float *Px = P + SX * PS + row;
                         const float du = d1_taps<M>(c, [&](int t) { return Rw[t]; }, g.inv_dx);
                         const float dpsi = d1_taps<M>(c, [&](int t) { return Px[t]; }, g.inv_dx);
                         const float psi0 = cpx[r];
-                        const float tmp = ((1.0f + bx) * lx + dbx * du) + ax * dpsi + dax * psi0;
                         const float z0v = czx[r];
-                        w_sum += (1.0f + bx) * tmp + ax * z0v;
-                        pnx.st_nt(bx * du + ax * psi0, col[r], so);
-                        zex.st_nt(bx * tmp + ax * z0v, col[r], so);
+                        w_sum += cpml_axis<BIG>(lx, ax, bx, dbx, dax, du, dpsi, psi0, z0v, psi1, z1v);
+                        pnx.st(psi1, col[r], so);
+                        zex.st(z1v, col[r], so);
                     } else {
                         w_sum += lx;
                     }
@@ -447,13 +516,12 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4)
                         const float du = d1_taps<M>(c, [&](int t) { return Rw[t * LW]; }, g.inv_dy);
                         const float dpsi = d1_taps<M>(c, [&](int t) { return Py[t * LW]; }, g.inv_dy);
                         const float psi0 = cpy[r];
-                        const float tmp = ((1.0f + by[r]) * ly + dby[r] * du) + ay[r] * dpsi + day[r] * psi0;
                         const float z0v = czy[r];
-                        w_sum += (1.0f + by[r]) * tmp + ay[r] * z0v;
-                        pny.st_nt(by[r] * du + ay[r] * psi0, col[r], so);
-                        zey.st_nt(by[r] * tmp + ay[r] * z0v, col[r], so);
+                        w_sum += cpml_axis<BIG && (BX || BZ)>(ly, ay[r], by[r], dby[r], day[r], du, dpsi, psi0, z0v, psi1, z1v);
+                        pny.st(psi1, col[r], so);
+                        zey.st(z1v, col[r], so);
                     } else {
-                        w_sum += ly;
+                        w_sum = fd::plus_scaled<TAIL_Y>(w_sum, acc_y, g.inv_dy2);
                     }
                     if constexpr (BZ) {
                         if (bandz) {
@@ -461,21 +529,20 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4)
                             const float du = d1_taps<M>(c, qz, g.inv_dz);
                             const float dpsi = d1_taps<M>(c, qpz, g.inv_dz);
                             const float psi0 = qp[r][C];
-                            const float tmp = ((1.0f + bz) * lz + dbz * du) + az * dpsi + daz * psi0;
                             const float z0v = czz[r];
-                            w_sum += (1.0f + bz) * tmp + az * z0v;
-                            pnz.st_nt(bz * du + az * psi0, col[r], so);
-                            zez.st_nt(bz * tmp + az * z0v, col[r], so);
+                            w_sum += cpml_axis<false>(lz, az, bz, dbz, daz, du, dpsi, psi0, z0v, psi1, z1v);
+                            pnz.st(psi1, col[r], so);
+                            zez.st(z1v, col[r], so);
                         } else {
-                            w_sum += lz;
+                            w_sum = fd::plus_scaled<TAIL_Z>(w_sum, acc_z, g.inv_dz2);
                         }
                     } else {
-                        w_sum += lz;
+                        w_sum = fd::plus_scaled<TAIL_Z>(w_sum, acc_z, g.inv_dz2);
                     }
                 }
             }
             const float v = cv[r];
-            unx.st_nt(2.0f * u0 - cup[r] + (v * v) * dt * dt * w_sum, col[r], so);
+            unx.st(fd::fused((v * v) * dt * dt, w_sum, 2.0f * u0 - cup[r]), col[r], so);
             if (u_this) u_this[off + int64_t(z) * sxy + col[r] / 4u] = (v * v) * w_sum;
         }
         if (z + 1 < ze) store_plane(lds[(S + 1) & 1], (C + 1) % R, (S + 1) % H);
@@ -499,20 +566,23 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4)
 // -- the expression tree of the per-cell adjoint (adjoint_split.cu:56-318)
 // with each neighbour's T formed once.  img != nullptr fuses the lagged
 // full-mode imaging grad += 2 dt^2 img lambda / v.
+template <int M, int RY, bool BX, bool BY, int NW>
+constexpr int adj_plane() { return (1 + (BX ? 3 : 0) + (BY ? 3 : 0)) * (NW * RY + 2 * M) * (64 + 2 * M); }
+
 template <int M, int RY, bool BX, bool BY, bool BZ, int NW>
-__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 8 ? 4 : 1))) adj3_kernel(Geo g, Coef c, Prof pr, AdjFields f, const float *__restrict__ img, float *__restrict__ grad, ZSet zs)
+__device__ __forceinline__ void adj3_tile(const Geo &g, const Coef &c, const Prof &pr, const AdjFields &f,
+                                          const float *__restrict__ img, float *__restrict__ grad, const ZTile &tile,
+                                          float *lds_mem)
 {
     constexpr bool SHELL = BX || BY || BZ;
     constexpr int TY = NW * RY;
     using PM = PlaneMap<M, TY, NW>;
     constexpr int LW = PM::LW, PS = PM::LH * PM::LW, YH = PM::YH;
-    constexpr int NPL = 1 + (BX ? 3 : 0) + (BY ? 3 : 0);
     constexpr int SX = 1, SY = BX ? 4 : 1;   // first plane slot of (U, V, W) for x, y
     constexpr int R = 2 * M + 2, H = M + 1;
-    __shared__ float lds[2][NPL * PS];
-    int b, k, xo, yo, zb, ze;
-    if (!zcoords<TY>(zs, b, k, xo, yo, zb, ze)) return;
-    const ZRect Rc = zs.r[k];
+    float *const lds[2] = {lds_mem, lds_mem + adj_plane<M, RY, BX, BY, NW>()};
+    const int b = tile.b, xo = tile.xo, yo = tile.yo, zb = tile.zb, ze = tile.ze;
+    const ZRect &Rc = tile.r;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int nx = g.nx, ny = g.ny;
     const int64_t sxy = g.sxy;
@@ -523,15 +593,15 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
     const float dt2 = g.dt2;
     // fields from plane zb - M on; plane z sits at byte offset pl(z)
     const int zbase = zb - M;
-    const int64_t fb = off + int64_t(zbase) * sxy, fe = off + g.n;
-    const int64_t mb = int64_t(b) * g.mstride + int64_t(zbase) * sxy, me = int64_t(b) * g.mstride + g.n;
+    const int64_t fb = off + int64_t(zbase) * sxy;
+    const int64_t mb = int64_t(b) * g.mstride + int64_t(zbase) * sxy;
     const uint32_t sxy4 = uint32_t(sxy) * 4u;
     auto pl = [&](int z) { return uint32_t(z - zbase) * sxy4; };
-    const Fld ln(f.l_now, fb, fe), lp(f.l_prev, fb, fe), lnx(f.l_next, fb, fe), vp(f.vp, mb, me);
-    const Fld psx(f.psi[0], fb, fe), psy(f.psi[1], fb, fe), psz(f.psi[2], fb, fe);
-    const Fld zex(f.zeta[0], fb, fe), zey(f.zeta[1], fb, fe), zez(f.zeta[2], fb, fe);
-    const Fld pox(f.psio[0], fb, fe), poy(f.psio[1], fb, fe), poz(f.psio[2], fb, fe);
-    const Fld zox(f.zetao[0], fb, fe), zoy(f.zetao[1], fb, fe), zoz(f.zetao[2], fb, fe);
+    const Ptr ln(f.l_now, fb), lp(f.l_prev, fb), lnx(f.l_next, fb), vp(f.vp, mb);
+    const Ptr psx(f.psi[0], fb), psy(f.psi[1], fb), psz(f.psi[2], fb);
+    const Ptr zex(f.zeta[0], fb), zey(f.zeta[1], fb), zez(f.zeta[2], fb);
+    const Ptr pox(f.psio[0], fb), poy(f.psio[1], fb), poz(f.psio[2], fb);
+    const Ptr zox(f.zetao[0], fb), zoy(f.zetao[1], fb), zoz(f.zetao[2], fb);
 
     uint32_t col[RY], yhc[YH];   // in-plane byte offsets
 #pragma unroll
@@ -597,8 +667,8 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
             nl[r] = ln.ld(col[r], so);
             nvh[r] = vp.ld(col[r], so);
             if constexpr (BZ) {
-                nzh[r] = zez.ld_nt(col[r], so);
-                nph[r] = psz.ld_nt(col[r], so);
+                nzh[r] = zez.ld(col[r], so);
+                nph[r] = psz.ld(col[r], so);
             }
         }
         if (xh.lds >= 0) {
@@ -635,7 +705,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
         const uint32_t so = pl(zn);
 #pragma unroll
         for (int r = 0; r < RY; ++r) {
-            nlp[r] = lp.ld_nt(col[r], so);
+            nlp[r] = lp.ld(col[r], so);
             if constexpr (BX) {
                 nzx[r] = zex.ld(col[r], so);
                 npx[r] = psx.ld(col[r], so);
@@ -793,8 +863,8 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
                     Lt[0] = Ls * g.inv_dx2.inv;
                     Dg[0] = Dgg * g.inv_dx.inv;
                     Dq *= g.inv_dx.inv;
-                    pox.st_nt(ax * cpx[r] + dax * gt0 - Dq, col[r], so);
-                    zox.st_nt(ax * (czx[r] + gw), col[r], so);
+                    pox.st(ax * cpx[r] + dax * gt0 - Dq, col[r], so);
+                    zox.st(ax * (czx[r] + gw), col[r], so);
                 } else {
                     float Ls = 0.f;
 #pragma unroll
@@ -816,8 +886,8 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
                     Lt[1] = Ls * g.inv_dy2.inv;
                     Dg[1] = Dgg * g.inv_dy.inv;
                     Dq *= g.inv_dy.inv;
-                    poy.st_nt(ay[r] * cpy[r] + day[r] * gt0 - Dq, col[r], so);
-                    zoy.st_nt(ay[r] * (czy[r] + gw), col[r], so);
+                    poy.st(ay[r] * cpy[r] + day[r] * gt0 - Dq, col[r], so);
+                    zoy.st(ay[r] * (czy[r] + gw), col[r], so);
                 } else {
                     float Ls = 0.f;
 #pragma unroll
@@ -838,8 +908,8 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
                     Lt[2] = Ls * g.inv_dz2.inv;
                     Dg[2] = Dgg * g.inv_dz.inv;
                     Dq *= g.inv_dz.inv;
-                    poz.st_nt(az * cpz[r] + daz * gt0 - Dq, col[r], so);
-                    zoz.st_nt(az * (czz[r] + gw), col[r], so);
+                    poz.st(az * cpz[r] + daz * gt0 - Dq, col[r], so);
+                    zoz.st(az * (czz[r] + gw), col[r], so);
                 } else {
                     float Ls = 0.f;
 #pragma unroll
@@ -849,13 +919,83 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
                 }
                 out = 2.0f * gun - clp[r] + (Lt[0] + Lt[1] + Lt[2] - Dg[0] - Dg[1] - Dg[2]);
             }
-            lnx.st_nt(out, col[r], so);
+            lnx.st(out, col[r], so);
         }
         push_head(zh, (S + 2 * M + 1) % R, S % H);
         if (z + 1 < ze) store_plane(lds[(S + 1) & 1], (C + 1) % R, (S + 1) % H);
         __syncthreads();
         return true;
         });
+    }
+}
+
+// ---------------------------------------------------------------- step kernels
+// Rows per lane and waves per workgroup of the reconstruction (a block's tile
+// is 64 x NW*RY cells; each plane re-reads 2M halo rows per tile, so a taller
+// tile of more waves cuts the y-halo share without more registers per lane).
+constexpr int kRyRecon = 4;
+constexpr int kNwRecon = 8;
+
+// Rows per lane of a region type (bits BX, BY, BZ); the step kernels run 4
+// waves a workgroup, so a tile is 64 x 4 ry_of(type) cells.
+constexpr int ry_of(int type)
+{
+    const int axes = (type & 1) + (type >> 1 & 1) + (type >> 2 & 1);
+    return axes == 0 ? 4 : axes == 1 ? 2 : 1;
+}
+
+template <int M, int T>
+constexpr int fwd_lds() { return fwd_plane<M, ry_of(T), (T & 1) != 0, (T & 2) != 0, 4>(); }
+template <int M, int T>
+constexpr int adj_lds() { return adj_plane<M, ry_of(T), (T & 1) != 0, (T & 2) != 0, 4>(); }
+constexpr int max4(int a, int b, int c, int d) { return std::max(std::max(a, b), std::max(c, d)); }
+
+template <int M, bool BIG>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+fwd3_kernel(Geo g, Coef c, Prof pr, StepFields f, float *__restrict__ u_this, float *__restrict__ strip, ZPlan zp)
+{
+    __shared__ float lds[2 * max4(fwd_lds<M, 0>(), fwd_lds<M, 1>(), fwd_lds<M, 2>(), fwd_lds<M, 3>())];
+    int type;
+    ZTile tile;
+    if (!zplan_tile(zp, g.B, type, tile)) return;
+    switch (type) {
+#define SWP_FWD3(T) \
+    case T: fwd3_tile<M, ry_of(T), (T & 1) != 0, (T & 2) != 0, (T & 4) != 0, 4, BIG>(g, c, pr, f, u_this, strip, tile, lds); break
+        SWP_FWD3(0);
+        SWP_FWD3(1);
+        SWP_FWD3(2);
+        SWP_FWD3(3);
+        SWP_FWD3(4);
+        SWP_FWD3(5);
+        SWP_FWD3(6);
+        SWP_FWD3(7);
+#undef SWP_FWD3
+    }
+}
+
+// Three waves per SIMD: left alone the widest type takes 212 VGPRs and two
+// (256 x 512 x 512, two shots, 100 steps: 571 against 556 ms; 97 x 110 x 131:
+// 47.9 against 44.3 ms).
+template <int M>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+adj3_kernel(Geo g, Coef c, Prof pr, AdjFields f, const float *__restrict__ img, float *__restrict__ grad, ZPlan zp)
+{
+    __shared__ float lds[2 * max4(adj_lds<M, 0>(), adj_lds<M, 1>(), adj_lds<M, 2>(), adj_lds<M, 3>())];
+    int type;
+    ZTile tile;
+    if (!zplan_tile(zp, g.B, type, tile)) return;
+    switch (type) {
+#define SWP_ADJ3(T) \
+    case T: adj3_tile<M, ry_of(T), (T & 1) != 0, (T & 2) != 0, (T & 4) != 0, 4>(g, c, pr, f, img, grad, tile, lds); break
+        SWP_ADJ3(0);
+        SWP_ADJ3(1);
+        SWP_ADJ3(2);
+        SWP_ADJ3(3);
+        SWP_ADJ3(4);
+        SWP_ADJ3(5);
+        SWP_ADJ3(6);
+        SWP_ADJ3(7);
+#undef SWP_ADJ3
     }
 }
 
@@ -872,9 +1012,10 @@ __global__ void __launch_bounds__(64 * NW) recon_zm_kernel(Geo g, Coef c, const 
     using PM = PlaneMap<M, TY, NW>;
     constexpr int LW = PM::LW;
     __shared__ float lds[2][PM::LH * PM::LW];
-    int b, k, xo, yo, zb, ze;
-    if (!zcoords<TY>(zs, b, k, xo, yo, zb, ze)) return;
-    const ZRect R = zs.r[k];
+    ZTile tile;
+    if (!zcoords<TY>(zs, tile)) return;
+    const ZRect &R = tile.r;
+    const int b = tile.b, xo = tile.xo, yo = tile.yo, zb = tile.zb, ze = tile.ze;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int nx = g.nx, ny = g.ny;
     const int64_t sxy = g.sxy;
@@ -887,8 +1028,8 @@ __global__ void __launch_bounds__(64 * NW) recon_zm_kernel(Geo g, Coef c, const 
     const int64_t mb = int64_t(b) * g.mstride + int64_t(zbase) * sxy, me = int64_t(b) * g.mstride + g.n;
     const uint32_t sxy4 = uint32_t(sxy) * 4u;
     auto pl = [&](int z) { return uint32_t(z - zbase) * sxy4; };
-    const Fld un(u_now, fb, fe), up(u_prev, fb, fe), unx(u_next, fb, fe), vp(vpb, mb, me);
-    const Fld ad(adj, fb, fe), gr(grad, fb, fe);   // unused without grad
+    const Buf un(u_now, fb, fe), up(u_prev, fb, fe), unx(u_next, fb, fe), vp(vpb, mb, me);
+    const Buf ad(adj, fb, fe), gr(grad, fb, fe);   // unused without grad
     const bool img_x = L.x >= g.X0 + g.W && L.x < g.X1 - g.W;
     bool img_y[RY];
     uint32_t col[RY], xhc[RY], yhc[PM::YH];   // in-plane byte offsets
@@ -992,17 +1133,6 @@ __global__ void __launch_bounds__(64 * NW) recon_zm_kernel(Geo g, Coef c, const 
 }
 
 // ---------------------------------------------------------------- host plans
-// Rows per lane and waves per workgroup of the interior kernels (a block's
-// tile is 64 x NW*RY cells; each plane re-reads 2M halo rows per tile, so a
-// taller tile of more waves cuts the y-halo share without more registers per
-// lane).  The margin kernels keep 4 waves.
-constexpr int kRyFwd = 4;
-constexpr int kRyAdj = 4;
-constexpr int kRyRecon = 4;
-constexpr int kNwFwd = 8;
-constexpr int kNwAdj = 4;
-constexpr int kNwRecon = 8;
-
 ZRect make_rect(int x0, int x1, int y0, int y1, int z0, int z1, int tz, int TY, int px)
 {
     ZRect R{};
@@ -1087,25 +1217,6 @@ void by_order(int M, K &&k)
     }
 }
 
-// The region set with its segment height: tz, halved (down to 16 planes)
-// while the launch would have fewer than `min_waves` waves (default 4096, 16
-// per CU; SWP_REGION_WAVES overrides, 1 keeps tz).  A block walks its
-// segment one plane (one load latency) at a time, so a region of few blocks
-// -- the edges and corners of the CPML margins -- runs for about tz plane
-// latencies however few cells it holds; shorter segments give it more
-// blocks that march fewer planes, at the cost of more 2M + 1 plane segment
-// prologues (which the larger regions avoid).
-ZSet region_set_sized(const Geo &g, bool ex, bool ey, bool ez, int tz, int TY, int NW)
-{
-    const int64_t min_waves = tuning(-1, "SWP_REGION_WAVES", 4096);
-    ZSet s = region_set(g, ex, ey, ez, tz, TY);
-    while (tz > 16 && int64_t(s.per_shot) * g.B * NW < min_waves) {
-        tz /= 2;
-        s = region_set(g, ex, ey, ez, tz, TY);
-    }
-    return s;
-}
-
 dim3 grid_of(const ZSet &s, int B)
 {
     const int64_t n = int64_t(s.per_shot) * B;
@@ -1113,42 +1224,48 @@ dim3 grid_of(const ZSet &s, int B)
     return dim3(unsigned(n));
 }
 
-// Rows per lane of the margin kernels, by the number of axes they carry.
-template <bool BX, bool BY, bool BZ>
-constexpr int ry_fwd() { return (int(BX) + int(BY) + int(BZ)) <= 1 ? 2 : 1; }
-template <bool BX, bool BY, bool BZ>
-constexpr int ry_adj() { return (int(BX) + int(BY) + int(BZ)) <= 1 ? 2 : 1; }
-
-template <int M, bool BX, bool BY, bool BZ>
-void fwd_region(const Ctx &x, const StepFields &f, float *u_this, float *strip)
+void census_region(const char *what, int type, int64_t blocks)
 {
-    constexpr bool SHELL = BX || BY || BZ;
-    constexpr int RY = SHELL ? ry_fwd<BX, BY, BZ>() : kRyFwd;
-    constexpr int NW = SHELL ? 4 : kNwFwd;
-    const ZSet s = region_set_sized(x.g, BX, BY, BZ, x.tz, NW * RY, NW);
-    if (!s.per_shot) return;
-    if (census_on()) {
-        const char site[] = {'a', '3', 'd', '.', 'f', 'w', 'd', '3', '.', char('0' + BX), char('0' + BY), char('0' + BZ), 0};
-        census_add(site, int64_t(s.per_shot) * x.g.B);
-    }
-    hipLaunchKernelGGL((fwd3_kernel<M, RY, BX, BY, BZ, NW>), grid_of(s, x.g.B), dim3(64 * NW), 0, stream(), x.g, x.c, x.pr,
-                       f, u_this, strip, s);
+    if (!census_on() || !blocks) return;
+    const char site[] = {'a', '3', 'd', '.', what[0], what[1], what[2], '3', '.', char('0' + (type & 1)),
+                         char('0' + (type >> 1 & 1)), char('0' + (type >> 2 & 1)), 0};
+    census_add(site, blocks);
 }
 
-template <int M, bool BX, bool BY, bool BZ>
-void adj_region(const Ctx &x, const AdjFields &f, const float *img, float *grad)
+// Segment height of a launch: tz, halved (down to kMinTz planes) while the
+// launch would have fewer than kMinWaves waves (SWP_REGION_WAVES overrides, 1
+// keeps tz).  A workgroup walks its segment one plane (one load latency) at a
+// time, so a launch of few workgroups takes about tz plane latencies however
+// few cells it holds; a shorter segment repeats its 2M + 1 plane prologue more
+// often.  Measured per gradient at 40 x 36 x 44 (two shots, order 4), 97 x 110
+// x 131 and, records only, 128 x 256 x 256 (order 8): 8 planes / 16384 waves
+// 41.5, 41.8 and 35.7 ms; 16 planes / 8192 waves 43.7, 44.6 and 36.2 ms.
+constexpr int64_t kMinWaves = 16384;
+constexpr int kMinTz = 8;
+
+// The plan of the region types in `mask` (bit t: type t).
+ZPlan make_zplan(const Geo &g, unsigned mask, int tz)
 {
-    constexpr bool SHELL = BX || BY || BZ;
-    constexpr int RY = SHELL ? ry_adj<BX, BY, BZ>() : kRyAdj;
-    constexpr int NW = SHELL ? 4 : kNwAdj;
-    const ZSet s = region_set_sized(x.g, BX, BY, BZ, x.tz, NW * RY, NW);
-    if (!s.per_shot) return;
-    if (census_on()) {
-        const char site[] = {'a', '3', 'd', '.', 'a', 'd', 'j', '3', '.', char('0' + BX), char('0' + BY), char('0' + BZ), 0};
-        census_add(site, int64_t(s.per_shot) * x.g.B);
+    const int64_t min_waves = tuning(-1, "SWP_REGION_WAVES", kMinWaves);
+    for (;; tz /= 2) {
+        ZPlan p{};
+        int64_t blocks = 0;
+        for (int t : {7, 3, 5, 6, 1, 2, 4, 0}) {
+            if (!(mask >> t & 1)) continue;
+            const ZSet s = region_set(g, t & 1, t & 2, t & 4, tz, 4 * ry_of(t));
+            if (!s.per_shot) continue;
+            const int k = p.n++;
+            p.type[k] = t;
+            p.ty[k] = 4 * ry_of(t);
+            p.per_shot[k] = s.per_shot;
+            for (int j = 0; j < s.n; ++j) p.r[p.r0[k] + j] = s.r[j];
+            p.r0[k + 1] = p.r0[k] + s.n;
+            blocks += (int64_t(s.per_shot) * g.B + 7) / 8 * 8;
+            SWP_CHECK(blocks < (int64_t(1) << 31), "acoustic3d: launch too large");
+            p.first[k + 1] = int(blocks);
+        }
+        if (tz <= kMinTz || blocks * 4 >= min_waves) return p;
     }
-    hipLaunchKernelGGL((adj3_kernel<M, RY, BX, BY, BZ, NW>), grid_of(s, x.g.B), dim3(64 * NW), 0, stream(), x.g, x.c, x.pr,
-                       f, img, grad, s);
 }
 
 }  // namespace
@@ -1180,36 +1297,27 @@ int shell_boxes(const Geo &g, Box out[6])
 
 void launch_fwd_zm(const Ctx &x, const StepFields &f, float *u_this, float *strip, bool shell)
 {
-    by_order(x.g.M, [&](auto ms) {
+    const Geo &g = x.g;
+    const ZPlan p = make_zplan(g, shell ? 0xffu : 1u, x.tz);
+    if (!p.n) return;
+    for (int k = 0; k < p.n; ++k) census_region("fwd", p.type[k], int64_t(p.per_shot[k]) * g.B);
+    by_order(g.M, [&](auto ms) {
         constexpr int M = decltype(ms)::value;
-        if (shell) {
-            fwd_region<M, true, true, true>(x, f, u_this, strip);
-            fwd_region<M, true, true, false>(x, f, u_this, strip);
-            fwd_region<M, true, false, true>(x, f, u_this, strip);
-            fwd_region<M, false, true, true>(x, f, u_this, strip);
-            fwd_region<M, true, false, false>(x, f, u_this, strip);
-            fwd_region<M, false, true, false>(x, f, u_this, strip);
-            fwd_region<M, false, false, true>(x, f, u_this, strip);
-        }
-        fwd_region<M, false, false, false>(x, f, u_this, strip);
+        hipLaunchKernelGGL((x.big ? fwd3_kernel<M, true> : fwd3_kernel<M, false>), dim3(unsigned(p.first[p.n])), dim3(256),
+                           0, stream(), g, x.c, x.pr, f, u_this, strip, p);
     });
     SWP_LAUNCHED();
 }
 
 void launch_adj_zm(const Ctx &x, const AdjFields &f, const float *img, float *grad, bool shell)
 {
-    by_order(x.g.M, [&](auto ms) {
-        constexpr int M = decltype(ms)::value;
-        if (shell) {
-            adj_region<M, true, true, true>(x, f, img, grad);
-            adj_region<M, true, true, false>(x, f, img, grad);
-            adj_region<M, true, false, true>(x, f, img, grad);
-            adj_region<M, false, true, true>(x, f, img, grad);
-            adj_region<M, true, false, false>(x, f, img, grad);
-            adj_region<M, false, true, false>(x, f, img, grad);
-            adj_region<M, false, false, true>(x, f, img, grad);
-        }
-        adj_region<M, false, false, false>(x, f, img, grad);
+    const Geo &g = x.g;
+    const ZPlan p = make_zplan(g, shell ? 0xffu : 1u, x.tz);
+    if (!p.n) return;
+    for (int k = 0; k < p.n; ++k) census_region("adj", p.type[k], int64_t(p.per_shot[k]) * g.B);
+    by_order(g.M, [&](auto ms) {
+        hipLaunchKernelGGL(adj3_kernel<decltype(ms)::value>, dim3(unsigned(p.first[p.n])), dim3(256), 0, stream(), g,
+                           x.c, x.pr, f, img, grad, p);
     });
     SWP_LAUNCHED();
 }
@@ -1218,9 +1326,15 @@ void launch_recon_zm(const Ctx &x, const float *vp, const float *u_prev, const f
                      const float *adj, float *grad, int x0, int x1, int y0, int y1, int z0, int z1)
 {
     const Geo &g = x.g;
-    ZSet s{};
-    add_rect(s, x0, x1, y0, y1, z0, z1, x.tz, kNwRecon * kRyRecon, x.g.px);
-    if (!s.per_shot) return;
+    const int64_t min_waves = tuning(-1, "SWP_REGION_WAVES", kMinWaves);
+    ZSet s;
+    int tz = x.tz;
+    do {
+        s = ZSet{};
+        add_rect(s, x0, x1, y0, y1, z0, z1, tz, kNwRecon * kRyRecon, x.g.px);
+        if (!s.per_shot) return;
+        tz /= 2;
+    } while (tz >= kMinTz && int64_t(s.per_shot) * g.B * kNwRecon < min_waves);
     census_add("a3d.recon_zm", int64_t(s.per_shot) * g.B);
     by_order(g.M, [&](auto ms) {
         constexpr int M = decltype(ms)::value;

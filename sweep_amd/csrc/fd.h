@@ -39,6 +39,36 @@ __device__ __forceinline__ float scaled_half(float a, Scale s)
 #endif
 }
 
+// a * b + c in one rounding, where a kernel fixes which product of a sum is
+// fused instead of leaving it to the compiler (the parity build rounds both).
+__device__ __forceinline__ float fused(float a, float b, float c)
+{
+#ifdef SWP_EXACT_DIV
+    return a * b + c;
+#else
+    return __builtin_fmaf(a, b, c);
+#endif
+}
+
+// x as rounded here: no operation on it is fused into the next one.
+__device__ __forceinline__ float rounded(float x)
+{
+    asm("" : "+v"(x));
+    return x;
+}
+
+// w + acc * (the scale): the product fused into the sum, or rounded first.
+template <bool FUSE>
+__device__ __forceinline__ float plus_scaled(float w, float acc, Scale s)
+{
+    if constexpr (FUSE) {
+#ifndef SWP_EXACT_DIV
+        return __builtin_fmaf(acc, s.inv, w);
+#endif
+    }
+    return w + rounded(scaled(acc, s));
+}
+
 // Forward second derivative: order 4 in summed form, the other fixed orders
 // in difference form (csrc/cuda/operators/laplace.cuh:68-387).
 template <int M, class C, class T, class S>
