@@ -11,10 +11,9 @@
 // tap: one 16-byte load from the NHWC input and one from the weights.
 //
 // The weight gradient reduces over pixels, which are not contiguous in
-// either operand, so each 32-pixel chunk of dout and of the tap-shifted
-// input is staged through LDS transposed to [channel][pixel]; the pixel
-// range is split across workgroups and the float32 partial tiles are summed
-// in a fixed order by a second kernel.
+// either operand; its transposing LDS reads are described at its kernel.  The
+// pixel range is split across workgroups and the float32 partial tiles are
+// summed in a fixed order by a second kernel.
 #include "unet.h"
 
 #include <algorithm>
@@ -118,100 +117,202 @@ __global__ void __launch_bounds__(256) conv_fwd_kernel(const uint16_t *__restric
 }
 
 // ---------------------------------------------------------------- weight gradient
-// Block: 64 (co) x 64 (ci) for one tap over one pixel split; wave wv owns
-// the 32 x 32 sub-tile (co (wv / 2) * 32, ci (wv % 2) * 32).
-// Grid: (ceil(cin / 64), ceil(cout / 64), ks * ks * splits).
-constexpr int kCP = 64;   // pixels per LDS chunk (two 32-pixel MFMA k-steps)
-constexpr int kLP = 72;   // LDS row pitch (bf16): kCP pixels + 8, 16-byte aligned rows
+// Block: 4 waves, 32 TO output x 32 TI input channels, every tap, over a strip
+// of SP columns and a segment of rows of one image.  The contraction runs over
+// pixels: each image row of the strip (input with its ks / 2 halo columns, dout
+// without) is staged once in LDS as [pixel][channel] and feeds all ks * ks taps
+// (the input rows of a window stay in a ring), where ds_read_b64_tr_b16 hands a
+// lane four pixels of its channel: a 16-lane group reads 4 pixels x 16 channels
+// and gets them transposed.  The same pixel order in both operands is all the
+// product needs, so lane group g takes pixels 4g.. and 16 + 4g.. of a 32-pixel
+// step, and a tap's shift is a pixel offset.  A wave owns a 32 x 32 channel tile
+// of all taps (144 accumulators at 3 x 3); a block of fewer than four channel
+// tiles gives the other waves (WK) pixels of their own.  Row pitches of 80 and 48
+// halves put 8 consecutive pixels' 32 bytes on different banks.  The next rows'
+// loads are in flight while a row is multiplied, one barrier a row.
+//
+// Measured in a 2 x 384 x 1152, 4-level, base-32 training step (14 layers, 285
+// GFLOP): 22 to 83 us a layer, 33.5 us on average at 64 x 64 tiles; one block a
+// tap, each staging both operands again through 2-byte transposing LDS stores,
+// took 395 us on average.  Bound by the LDS reads (80 transposing reads a wave
+// and row against 72 MFMAs).
+template <int KS, int TO, int TI>
+struct WgradTile {
+    static constexpr int WK = 4 / (TO * TI);
+    static constexpr int KPW = WK == 1 ? 64 : 32;    // pixels a wave takes of a row
+    static constexpr int SP = KPW * WK;              // strip columns
+    static constexpr int R = KS / 2;
+    static constexpr int NS = KS == 3 ? 4 : 2;       // input rows kept
+    static constexpr int PI = TI == 2 ? 80 : 48, PD = TO == 2 ? 80 : 48;
+    static constexpr int IW = SP + 2 * R;
+    static constexpr int UI = (IW * TI * 4 + 255) / 256, UD = (SP * TO * 4 + 255) / 256;   // 16-byte units a thread
+};
 
-template <int KS>
-__global__ void __launch_bounds__(256) wgrad_kernel(const uint16_t *__restrict__ in, int H, int W, int cin, int is,
-                                                    const uint16_t *__restrict__ dout, int cout, int ds,
-                                                    float *__restrict__ partials, int splits, int64_t P,
-                                                    int64_t per)
+typedef __attribute__((__vector_size__(4 * sizeof(short)))) short s16x4;
+
+__device__ __forceinline__ bf16x8 ld_tr(const uint16_t *p, int pitch)
 {
-    __shared__ __attribute__((aligned(16))) uint16_t sD[64 * kLP];
-    __shared__ __attribute__((aligned(16))) uint16_t sI[64 * kLP];
+    struct Pair {
+        s16x4 lo, hi;
+    } v;
+    using L = __attribute__((address_space(3))) s16x4;
+    v.lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((L *)(p));
+    v.hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((L *)(p + 16 * pitch));
+    return __builtin_bit_cast(bf16x8, v);
+}
+
+template <int KS, int TO, int TI>
+__global__ void __launch_bounds__(256, 2) wgrad_kernel(const uint16_t *__restrict__ in, int H, int W, int cin, int is,
+                                                       const uint16_t *__restrict__ dout, int cout, int ds,
+                                                       float *__restrict__ partials, int nsx, int nsy, int rows)
+{
+    using T = WgradTile<KS, TO, TI>;
+    __shared__ __attribute__((aligned(16))) uint16_t mem[T::NS * T::IW * T::PI + 2 * T::SP * T::PD];
+    auto sI = [&](int y) { return mem + (y + T::NS) % T::NS * (T::IW * T::PI); };
+    auto sD = [&](int y) { return mem + T::NS * T::IW * T::PI + (y & 1) * (T::SP * T::PD); };
     const int tid = int(threadIdx.x), lane = tid & 63, wv = tid >> 6;
-    const int r16 = lane & 15, g = lane >> 4;
-    const int ci0 = int(blockIdx.x) * 64, co0 = int(blockIdx.y) * 64;
-    const int tap = int(blockIdx.z) % (KS * KS), split = int(blockIdx.z) / (KS * KS);
-    const int dy = tap / KS - KS / 2, dx = tap % KS - KS / 2;
-    const int64_t pb = int64_t(split) * per, pe = std::min(P, pb + per);
-    const int wco = (wv >> 1) * 32, wci = (wv & 1) * 32;
-    const int lp = tid >> 3, lc = (tid & 7) * 8;
-    const int64_t HW = int64_t(H) * W;
-    f32x4 acc[2][2];
+    const int g = lane >> 4, i16 = lane & 15;
+    const int ci0 = int(blockIdx.y) * 32 * TI, co0 = int(blockIdx.z) * 32 * TO;
+    const int sx = int(blockIdx.x) % nsx, sy = int(blockIdx.x) / nsx % nsy, n = int(blockIdx.x) / (nsx * nsy);
+    const int x0 = sx * T::SP, yb = sy * rows, ye = std::min(yb + rows, H);
+    const int wk = wv / (TO * TI), wo = wv % (TO * TI) / TI, wi = wv % TI;
+
+    f32x4 acc[KS * KS][2][2];
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int t = 0; t < KS * KS; ++t)
 #pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int64_t p0 = pb; p0 < pe; p0 += kCP) {
+        for (int a = 0; a < 2; ++a)
 #pragma unroll
-        for (int h = 0; h < kCP / 32; ++h) {
-            const int pl = lp + 32 * h;
-            const int64_t p = p0 + pl;
-            u32x4 vd = {0u, 0u, 0u, 0u}, vi = {0u, 0u, 0u, 0u};
-            if (p < pe) {
-                if (co0 + lc < cout) vd = *reinterpret_cast<const u32x4 *>(dout + p * ds + co0 + lc);
-                if (ci0 + lc < cin) {
-                    const int64_t nn = p / HW, rem = p % HW;
-                    const int sy = int(rem / W) + dy, sx = int(rem % W) + dx;
-                    if (sy >= 0 && sy < H && sx >= 0 && sx < W)
-                        vi = *reinterpret_cast<const u32x4 *>(in + ((nn * H + sy) * W + sx) * is + ci0 + lc);
+            for (int b = 0; b < 2; ++b) acc[t][a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    u32x4 ri[T::UI], rd[T::UD];
+    auto fetch_in = [&](int y) {   // input row y (zeros outside the image)
+#pragma unroll
+        for (int u = 0; u < T::UI; ++u) {
+            const int k = tid + 256 * u, px = k / (TI * 4), c = ci0 + k % (TI * 4) * 8, x = x0 - T::R + px;
+            ri[u] = u32x4{0u, 0u, 0u, 0u};
+            if (px < T::IW && c < cin && y >= 0 && y < H && x >= 0 && x < W)
+                ri[u] = *reinterpret_cast<const u32x4 *>(in + ((int64_t(n) * H + y) * W + x) * is + c);
+        }
+    };
+    auto fetch_dout = [&](int y) {
+#pragma unroll
+        for (int u = 0; u < T::UD; ++u) {
+            const int k = tid + 256 * u, px = k / (TO * 4), c = co0 + k % (TO * 4) * 8, x = x0 + px;
+            rd[u] = u32x4{0u, 0u, 0u, 0u};
+            if (px < T::SP && c < cout && y < ye && x < W)
+                rd[u] = *reinterpret_cast<const u32x4 *>(dout + ((int64_t(n) * H + y) * W + x) * ds + c);
+        }
+    };
+    auto put_in = [&](int y) {
+        uint16_t *d = sI(y);
+#pragma unroll
+        for (int u = 0; u < T::UI; ++u) {
+            const int k = tid + 256 * u, px = k / (TI * 4);
+            if (px < T::IW) *reinterpret_cast<u32x4 *>(d + px * T::PI + k % (TI * 4) * 8) = ri[u];
+        }
+    };
+    auto put_dout = [&](int y) {
+        uint16_t *d = sD(y);
+#pragma unroll
+        for (int u = 0; u < T::UD; ++u) {
+            const int k = tid + 256 * u, px = k / (TO * 4);
+            if (px < T::SP) *reinterpret_cast<u32x4 *>(d + px * T::PD + k % (TO * 4) * 8) = rd[u];
+        }
+    };
+    for (int y = yb - T::R; y <= yb + T::R; ++y) {
+        fetch_in(y);
+        put_in(y);
+    }
+    fetch_dout(yb);
+    put_dout(yb);
+    const int fp = 4 * g + i16 / 4, fc = 4 * (i16 % 4);   // a lane's pixel and channel within a fragment
+    for (int y = yb; y < ye; ++y) {
+        __syncthreads();
+        fetch_in(y + T::R + 1);
+        fetch_dout(y + 1);
+#pragma unroll
+        for (int k = 0; k < T::KPW / 32; ++k) {
+            const int p = wk * T::KPW + 32 * k + fp;
+            bf16x8 A[2];
+#pragma unroll
+            for (int a = 0; a < 2; ++a) A[a] = ld_tr(sD(y) + p * T::PD + wo * 32 + 16 * a + fc, T::PD);
+#pragma unroll
+            for (int dy = 0; dy < KS; ++dy) {
+                const uint16_t *row = sI(y + dy - T::R) + wi * 32 + fc;
+#pragma unroll
+                for (int dx = 0; dx < KS; ++dx) {
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) {
+                        const bf16x8 Bv = ld_tr(row + (p + dx) * T::PI + 16 * b, T::PI);
+#pragma unroll
+                        for (int a = 0; a < 2; ++a) acc[dy * KS + dx][a][b] = mma(A[a], Bv, acc[dy * KS + dx][a][b]);
+                    }
                 }
             }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                sD[(lc + 2 * e) * kLP + pl] = uint16_t(vd[e] & 0xffffu);
-                sD[(lc + 2 * e + 1) * kLP + pl] = uint16_t(vd[e] >> 16);
-                sI[(lc + 2 * e) * kLP + pl] = uint16_t(vi[e] & 0xffffu);
-                sI[(lc + 2 * e + 1) * kLP + pl] = uint16_t(vi[e] >> 16);
-            }
         }
-        __syncthreads();
+        put_in(y + T::R + 1);
+        put_dout(y + 1);
+    }
+    // the waves of one channel tile (WK of them) meet in LDS, a tap at a time;
+    // each then writes 4 / WK of the tile's four 16 x 16 parts
+    f32x4 *red = reinterpret_cast<f32x4 *>(mem);
 #pragma unroll
-        for (int k = 0; k < kCP / 32; ++k) {
-            bf16x8 A[2], Bv[2];
-#pragma unroll
-            for (int a = 0; a < 2; ++a) A[a] = ld8(sD + (wco + 16 * a + r16) * kLP + 32 * k + 8 * g);
-#pragma unroll
-            for (int b = 0; b < 2; ++b) Bv[b] = ld8(sI + (wci + 16 * b + r16) * kLP + 32 * k + 8 * g);
+    for (int t = 0; t < KS * KS; ++t) {
+        float *dst = partials + (int64_t(blockIdx.x) * (KS * KS) + t) * cout * cin;
+        if constexpr (T::WK > 1) {
+            __syncthreads();
 #pragma unroll
             for (int a = 0; a < 2; ++a)
 #pragma unroll
-                for (int b = 0; b < 2; ++b) acc[a][b] = mma(A[a], Bv[b], acc[a][b]);
+                for (int b = 0; b < 2; ++b) red[(wv * 4 + 2 * a + b) * 64 + lane] = acc[t][a][b];
+            __syncthreads();
         }
-        __syncthreads();
-    }
-    float *dst = partials + (int64_t(split) * (KS * KS) + tap) * cout * cin;
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+        for (int a = 0; a < 2; ++a)
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            const int ci = ci0 + wci + 16 * b + r16;
-            if (ci >= cin) continue;
+            for (int b = 0; b < 2; ++b) {
+                f32x4 v = acc[t][a][b];
+                if constexpr (T::WK > 1) {
+                    if ((2 * a + b) % T::WK != wk) continue;
+                    v = red[((wv - wk * (TO * TI)) * 4 + 2 * a + b) * 64 + lane];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int co = co0 + wco + 16 * a + 4 * g + e;
-                if (co < cout) dst[int64_t(co) * cin + ci] = acc[a][b][e];
+                    for (int k = 1; k < T::WK; ++k) v += red[((wv + (k - wk) * (TO * TI)) * 4 + 2 * a + b) * 64 + lane];
+                }
+                const int ci = ci0 + wi * 32 + 16 * b + i16;
+                if (ci >= cin) continue;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int co = co0 + wo * 32 + 16 * a + 4 * g + e;
+                    if (co < cout) dst[int64_t(co) * cin + ci] = v[e];
+                }
             }
-        }
+    }
 }
 
-// dw[co, tap, ci] = sum over splits of partials[split, tap, co, ci].
+// dw[co, tap, ci] = sum over splits of partials[split, tap, co, ci].  A block
+// takes 32 consecutive values of the partials' order; its 8 groups of 32 lanes
+// stride the splits and meet in LDS, always in the same order.  (One thread a
+// value, walking up to 4096 splits alone, took 423 us a layer.)
 __global__ void __launch_bounds__(256) wgrad_reduce_kernel(const float *__restrict__ partials, int splits, int taps,
                                                            int cout, int cin, float *__restrict__ dw)
 {
+    __shared__ float red[256];
     const int64_t n = int64_t(taps) * cout * cin;
-    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += int64_t(gridDim.x) * 256) {
-        const int ci = int(i % cin);
-        const int64_t t2 = i / cin;
-        const int tap = int(t2 % taps), co = int(t2 / taps);
-        float s = 0.f;
-        for (int sp = 0; sp < splits; ++sp) s += partials[((int64_t(sp) * taps + tap) * cout + co) * cin + ci];
-        dw[i] = s;
+    const int64_t k = int64_t(blockIdx.x) * 32 + (threadIdx.x & 31);
+    float s = 0.f;
+    if (k < n) {
+#pragma unroll 4
+        for (int sp = int(threadIdx.x) >> 5; sp < splits; sp += 8) s += partials[int64_t(sp) * n + k];
     }
+    red[threadIdx.x] = s;
+    __syncthreads();
+    if (threadIdx.x >= 32 || k >= n) return;
+    for (int j = 1; j < 8; ++j) s += red[threadIdx.x + 32 * j];
+    const int ci = int(k % cin);
+    const int64_t t2 = k / cin;
+    const int co = int(t2 % cout), tap = int(t2 / cout);
+    dw[(int64_t(co) * taps + tap) * cin + ci] = s;
 }
 
 // partial[split, c] = sum over the split's pixels of x[p, c]; then out[c].
@@ -436,12 +537,26 @@ void check_view(const void *p, int stride, int channels, const char *what)
               ": channels (", channels, ") and stride (", stride, ") must be positive multiples of 8, channels <= stride");
 }
 
-int wgrad_splits(int64_t P, int cin, int cout, int ks)
+// The weight gradient's launch: 64 channels a tile where the count is a multiple
+// of 64, else 32; rows a segment so that at most 512 blocks run (two fit on
+// each of the 256 CUs) where that leaves at least 4.
+struct WgradPlan {
+    int to, ti, nsx, nsy, rows, blocks;
+};
+
+WgradPlan wgrad_plan(int N, int H, int W, int cin, int cout)
 {
-    const int64_t tiles = int64_t((cin + 63) / 64) * ((cout + 63) / 64) * ks * ks;
-    int64_t s = std::max<int64_t>(1, 2048 / tiles);
-    s = std::min<int64_t>(s, std::max<int64_t>(1, P / 256));
-    return int(std::min<int64_t>(s, 64));
+    WgradPlan p{};
+    p.to = cout % 64 == 0 ? 2 : 1;
+    p.ti = cin % 64 == 0 ? 2 : 1;
+    const int wk = 4 / (p.to * p.ti), sp = wk == 4 ? 128 : 64;
+    const int64_t tiles = int64_t((cin + 32 * p.ti - 1) / (32 * p.ti)) * ((cout + 32 * p.to - 1) / (32 * p.to));
+    p.nsx = (W + sp - 1) / sp;
+    const int64_t want = std::max<int64_t>(1, 512 / (tiles * p.nsx * N));
+    p.rows = int(std::max<int64_t>(std::min(H, 4), (H + want - 1) / want));
+    p.nsy = (H + p.rows - 1) / p.rows;
+    p.blocks = p.nsx * p.nsy * N;
+    return p;
 }
 
 constexpr int kColSplits = 512;
@@ -476,8 +591,7 @@ void conv_fwd(const uint16_t *in, int N, int H, int W, int cin, int in_stride, c
 
 int64_t conv_wgrad_partials(int N, int H, int W, int cin, int cout, int ks)
 {
-    const int64_t P = int64_t(N) * H * W;
-    return int64_t(wgrad_splits(P, cin, cout, ks)) * ks * ks * cout * cin + int64_t(kColSplits) * cout;
+    return int64_t(wgrad_plan(N, H, W, cin, cout).blocks) * ks * ks * cout * cin + int64_t(kColSplits) * cout;
 }
 
 void conv_wgrad(const uint16_t *in, int N, int H, int W, int cin, int in_stride, const uint16_t *dout, int cout,
@@ -489,19 +603,24 @@ void conv_wgrad(const uint16_t *in, int N, int H, int W, int cin, int in_stride,
     check_view(dout, dout_stride, cout, "wgrad dout");
     SWP_CHECK(dw && partials, "wgrad: null output or scratch");
     const int64_t P = int64_t(N) * H * W;
-    const int splits = wgrad_splits(P, cin, cout, ks);
-    int64_t per = (P + splits - 1) / splits;
-    per = (per + kCP - 1) / kCP * kCP;
-    const dim3 grid(unsigned((cin + 63) / 64), unsigned((cout + 63) / 64), unsigned(ks * ks * splits));
+    const WgradPlan w = wgrad_plan(N, H, W, cin, cout);
+    const int splits = w.blocks;
+    const dim3 grid(unsigned(w.blocks), unsigned((cin + 32 * w.ti - 1) / (32 * w.ti)),
+                    unsigned((cout + 32 * w.to - 1) / (32 * w.to)));
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream(), in, H, W, cin, in_stride, dout, cout, dout_stride,
+                           partials, w.nsx, w.nsy, w.rows);
+    };
+    const int tile = (w.to - 1) * 2 + w.ti - 1;
     if (ks == 3)
-        hipLaunchKernelGGL(wgrad_kernel<3>, grid, dim3(256), 0, stream(), in, H, W, cin, in_stride, dout, cout,
-                           dout_stride, partials, splits, P, per);
+        tile == 3 ? launch(wgrad_kernel<3, 2, 2>) : tile == 2 ? launch(wgrad_kernel<3, 2, 1>)
+            : tile == 1 ? launch(wgrad_kernel<3, 1, 2>) : launch(wgrad_kernel<3, 1, 1>);
     else
-        hipLaunchKernelGGL(wgrad_kernel<1>, grid, dim3(256), 0, stream(), in, H, W, cin, in_stride, dout, cout,
-                           dout_stride, partials, splits, P, per);
+        tile == 3 ? launch(wgrad_kernel<1, 2, 2>) : tile == 2 ? launch(wgrad_kernel<1, 2, 1>)
+            : tile == 1 ? launch(wgrad_kernel<1, 1, 2>) : launch(wgrad_kernel<1, 1, 1>);
     SWP_LAUNCHED();
     const int64_t n = int64_t(ks) * ks * cout * cin;
-    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(blocks_for(n)), dim3(256), 0, stream(), partials, splits, ks * ks,
+    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(unsigned((n + 31) / 32)), dim3(256), 0, stream(), partials, splits, ks * ks,
                        cout, cin, dw);
     SWP_LAUNCHED();
     if (db) {
