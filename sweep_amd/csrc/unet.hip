@@ -50,10 +50,138 @@ __device__ __forceinline__ f32x4 mma(bf16x8 a, bf16x8 b, f32x4 c)
 }
 
 // ---------------------------------------------------------------- forward
-// Block: 4 waves, 128 consecutive pixels of one image row (32 per wave, two
-// 16-row A tiles) x 64 output channels (four 16-column B tiles).
-// Grid: (ceil(W / 128), H, N * ceil(cout / 64)).
-template <int KS, bool F32OUT>
+// At most 32 input channels (one MFMA step a tap).  Block: 4 waves, 64 columns x
+// 4 rows of pixels (a row a wave) x 16 NT output channels.  The block stages its
+// pixels with their halo in LDS once for all taps, and the weights a row of taps
+// at a time; a wave's 4 x NT MFMAs of a tap then take 4 + NT fragments from LDS (16
+// bytes a lane, rows of 80 bytes: the 16 lanes of a group on 16 different bank
+// quads).  The weights are the first operand, so a lane ends up with four
+// consecutive channels of a pixel and stores them together.  The next phase's
+// global loads are in flight while a phase multiplies.
+// NT 4 from 33 channels up, 2 from 17, else 1: the network's 32- and 8-channel
+// layers multiplied 2 and 8 times their channels in tiles of 64.
+constexpr int kCPitch = 40;   // LDS row (32 channels of a pixel or weight row) in halves
+
+template <int KS, int NT, bool F32OUT>
+__global__ void __launch_bounds__(256, 2) conv_c32_kernel(const uint16_t *__restrict__ in, int H, int W, int cin,
+                                                          int is, const uint16_t *__restrict__ w, int cout,
+                                                          const float *__restrict__ bias, int relu,
+                                                          void *__restrict__ out, int os, int ncot, int vec)
+{
+    constexpr int R = KS / 2, IW = 64 + 2 * R, IH = 4 + 2 * R, CO = 16 * NT;
+    constexpr int UI = (IH * IW * 4 + 255) / 256, UW = (KS * CO * 4 + 255) / 256;   // 16-byte units a thread
+    __shared__ __attribute__((aligned(16))) uint16_t sI[IH * IW * kCPitch];
+    __shared__ __attribute__((aligned(16))) uint16_t sW[KS * CO * kCPitch];
+    const int tid = int(threadIdx.x), lane = tid & 63, wv = tid >> 6;
+    const int r16 = lane & 15, g = lane >> 4;
+    const int x0 = int(blockIdx.x) * 64, y0 = int(blockIdx.y) * 4;
+    const int n = int(blockIdx.z) / ncot, co0 = (int(blockIdx.z) % ncot) * CO;
+    f32x4 acc[4][NT];
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    u32x4 ri[UI], rw[UW];
+    auto fetch_in = [&] {   // the pixels and their halo (zeros outside)
+#pragma unroll
+        for (int u = 0; u < UI; ++u) {
+            const int k = tid + 256 * u, px = k >> 2, ci = (k & 3) * 8;
+            const int y = y0 - R + px / IW, x = x0 - R + px % IW;
+            ri[u] = u32x4{0u, 0u, 0u, 0u};
+            if (px < IH * IW && ci < cin && y >= 0 && y < H && x >= 0 && x < W)
+                ri[u] = *reinterpret_cast<const u32x4 *>(in + ((int64_t(n) * H + y) * W + x) * is + ci);
+        }
+    };
+    auto fetch_w = [&](int dy) {   // the KS taps of row dy
+#pragma unroll
+        for (int u = 0; u < UW; ++u) {
+            const int k = tid + 256 * u, row = k >> 2, ci = (k & 3) * 8;
+            const int dx = row / CO, co = co0 + row % CO;
+            rw[u] = u32x4{0u, 0u, 0u, 0u};
+            if (row < KS * CO && ci < cin && co < cout)
+                rw[u] = *reinterpret_cast<const u32x4 *>(w + (int64_t(co) * (KS * KS) + dy * KS + dx) * cin + ci);
+        }
+    };
+    fetch_in();
+    fetch_w(0);
+#pragma unroll
+    for (int dy = 0; dy < KS; ++dy) {
+        __syncthreads();
+        if (dy == 0) {
+#pragma unroll
+            for (int u = 0; u < UI; ++u) {
+                const int k = tid + 256 * u;
+                if (k < IH * IW * 4) *reinterpret_cast<u32x4 *>(sI + (k >> 2) * kCPitch + (k & 3) * 8) = ri[u];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < UW; ++u) {
+            const int k = tid + 256 * u;
+            if (k < KS * CO * 4) *reinterpret_cast<u32x4 *>(sW + (k >> 2) * kCPitch + (k & 3) * 8) = rw[u];
+        }
+        __syncthreads();
+        if (dy + 1 < KS) fetch_w(dy + 1);
+#pragma unroll
+        for (int dx = 0; dx < KS; ++dx) {
+            bf16x8 wf[NT], px[4];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) wf[t] = ld8(sW + (dx * CO + 16 * t + r16) * kCPitch + 8 * g);
+#pragma unroll
+            for (int m = 0; m < 4; ++m) px[m] = ld8(sI + ((wv + dy) * IW + 16 * m + r16 + dx) * kCPitch + 8 * g);
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) acc[m][t] = mma(wf[t], px[m], acc[m][t]);
+        }
+    }
+    const int y = y0 + wv;
+    if (y >= H) return;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int co = co0 + 16 * t + 4 * g;
+        if (co >= cout) continue;
+        float bv[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bv[e] = bias && co + e < cout ? bias[co + e] : 0.f;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            const int x = x0 + 16 * m + r16;
+            if (x >= W) continue;
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[e] = acc[m][t][e] + bv[e];
+                if (relu) v[e] = fmaxf(v[e], 0.f);
+            }
+            const int64_t i = ((int64_t(n) * H + y) * W + x) * os + co;
+            if (vec && co + 4 <= cout) {   // four channels in one store (out and os allow it)
+                if constexpr (F32OUT) {
+                    *reinterpret_cast<f32x4 *>(static_cast<float *>(out) + i) = f32x4{v[0], v[1], v[2], v[3]};
+                } else {
+                    typedef __attribute__((__vector_size__(2 * sizeof(uint32_t)))) uint32_t u32x2;
+                    *reinterpret_cast<u32x2 *>(static_cast<uint16_t *>(out) + i) =
+                        u32x2{uint32_t(f2bf(v[0])) | uint32_t(f2bf(v[1])) << 16,
+                              uint32_t(f2bf(v[2])) | uint32_t(f2bf(v[3])) << 16};
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (co + e >= cout) break;
+                    if constexpr (F32OUT) static_cast<float *>(out)[i + e] = v[e];
+                    else static_cast<uint16_t *>(out)[i + e] = f2bf(v[e]);
+                }
+            }
+        }
+    }
+}
+
+// More than 32 input channels.  Block: 4 waves, 128 consecutive pixels of one
+// image row (32 per wave, two 16-row A tiles) x 16 NT output channels.
+// Grid: (ceil(W / 128), H, N * ceil(cout / (16 NT))).  Every operand comes from
+// L1 or L2; staging a chunk of the input for all taps instead would sum the
+// chunks before the taps, and the network's bf16 activations then round apart.
+template <int KS, int NT, bool F32OUT>
 __global__ void __launch_bounds__(256) conv_fwd_kernel(const uint16_t *__restrict__ in, int H, int W, int cin,
                                                        int is, const uint16_t *__restrict__ w, int cout,
                                                        const float *__restrict__ bias, int relu,
@@ -62,15 +190,15 @@ __global__ void __launch_bounds__(256) conv_fwd_kernel(const uint16_t *__restric
     const int lane = int(threadIdx.x) & 63, wv = int(threadIdx.x) >> 6;
     const int r16 = lane & 15, g = lane >> 4;
     const int y = int(blockIdx.y);
-    const int n = int(blockIdx.z) / ncot, co0 = (int(blockIdx.z) % ncot) * 64;
+    const int n = int(blockIdx.z) / ncot, co0 = (int(blockIdx.z) % ncot) * 16 * NT;
     const int x0 = int(blockIdx.x) * 128 + wv * 32;
     constexpr int R = KS / 2;
     const int nchunk = (cin + 31) / 32;
-    f32x4 acc[2][4];
+    f32x4 acc[2][NT];
 #pragma unroll
     for (int m = 0; m < 2; ++m)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < NT; ++t) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int tap = 0; tap < KS * KS; ++tap) {
         const int sy = y + tap / KS - R, dx = tap % KS - R;
         const bool rowok = sy >= 0 && sy < H;
@@ -78,26 +206,26 @@ __global__ void __launch_bounds__(256) conv_fwd_kernel(const uint16_t *__restric
         for (int c = 0; c < nchunk; ++c) {
             const int ci = c * 32 + 8 * g;
             const bool ciok = ci < cin;
-            bf16x8 a[2], b[4];
+            bf16x8 a[2], b[NT];
 #pragma unroll
             for (int m = 0; m < 2; ++m) {
                 const int sx = x0 + 16 * m + r16 + dx;
                 a[m] = (rowok && ciok && sx >= 0 && sx < W) ? ld8(in + (rowbase + sx) * is + ci) : zero8();
             }
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
+            for (int t = 0; t < NT; ++t) {
                 const int co = co0 + 16 * t + r16;
                 b[t] = (ciok && co < cout) ? ld8(w + (int64_t(co) * (KS * KS) + tap) * cin + ci) : zero8();
             }
 #pragma unroll
             for (int m = 0; m < 2; ++m)
 #pragma unroll
-                for (int t = 0; t < 4; ++t) acc[m][t] = mma(a[m], b[t], acc[m][t]);
+                for (int t = 0; t < NT; ++t) acc[m][t] = mma(a[m], b[t], acc[m][t]);
         }
     }
     const int64_t obase = (int64_t(n) * H + y) * W;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
+    for (int t = 0; t < NT; ++t) {
         const int co = co0 + 16 * t + r16;
         if (co >= cout) continue;
         const float bv = bias ? bias[co] : 0.f;
@@ -572,19 +700,35 @@ void conv_fwd(const uint16_t *in, int N, int H, int W, int cin, int in_stride, c
     check_view(in, in_stride, cin, "conv input");
     SWP_CHECK(w && (reinterpret_cast<uintptr_t>(w) & 15) == 0, "conv: weights null or not 16-byte aligned");
     SWP_CHECK(out && cout >= 1 && cout <= out_stride, "conv: bad output view");
-    const int ncot = (cout + 63) / 64;
-    const dim3 grid(unsigned((W + 127) / 128), unsigned(H), unsigned(N * ncot));
+    const int nt = cout > 32 ? 4 : cout > 16 ? 2 : 1;
+    const int ncot = (cout + 16 * nt - 1) / (16 * nt);
     const int r = relu ? 1 : 0;
-#define SWP_CONV_LAUNCH(KS, F32)                                                                              \
-    hipLaunchKernelGGL((conv_fwd_kernel<KS, F32>), grid, dim3(256), 0, stream(), in, H, W, cin, in_stride, w, \
-                       cout, bias, r, out, out_stride, ncot)
+    const int vec = out_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & (out_f32 ? 15 : 7)) == 0;
+    const dim3 grid(unsigned((W + 127) / 128), unsigned(H), unsigned(N * ncot));
+    const dim3 grid32(unsigned((W + 63) / 64), unsigned((H + 3) / 4), unsigned(N * ncot));
+#define SWP_CONV_LAUNCH(KS, NT, F32)                                                                               \
+    do {                                                                                                           \
+        if (cin <= 32)                                                                                             \
+            hipLaunchKernelGGL((conv_c32_kernel<KS, NT, F32>), grid32, dim3(256), 0, stream(), in, H, W, cin,      \
+                               in_stride, w, cout, bias, r, out, out_stride, ncot, vec);                           \
+        else                                                                                                       \
+            hipLaunchKernelGGL((conv_fwd_kernel<KS, NT, F32>), grid, dim3(256), 0, stream(), in, H, W, cin,        \
+                               in_stride, w, cout, bias, r, out, out_stride, ncot);                                \
+    } while (0)
+#define SWP_CONV_NT(KS, F32)                         \
+    do {                                             \
+        if (nt == 4) SWP_CONV_LAUNCH(KS, 4, F32);    \
+        else if (nt == 2) SWP_CONV_LAUNCH(KS, 2, F32); \
+        else SWP_CONV_LAUNCH(KS, 1, F32);            \
+    } while (0)
     if (ks == 3) {
-        if (out_f32) SWP_CONV_LAUNCH(3, true);
-        else SWP_CONV_LAUNCH(3, false);
+        if (out_f32) SWP_CONV_NT(3, true);
+        else SWP_CONV_NT(3, false);
     } else {
-        if (out_f32) SWP_CONV_LAUNCH(1, true);
-        else SWP_CONV_LAUNCH(1, false);
+        if (out_f32) SWP_CONV_NT(1, true);
+        else SWP_CONV_NT(1, false);
     }
+#undef SWP_CONV_NT
 #undef SWP_CONV_LAUNCH
     SWP_LAUNCHED();
 }
