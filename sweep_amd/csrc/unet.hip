@@ -59,7 +59,8 @@ __device__ __forceinline__ f32x4 mma(bf16x8 a, bf16x8 b, f32x4 c)
 // consecutive channels of a pixel and stores them together.  The next phase's
 // global loads are in flight while a phase multiplies.
 // NT 4 from 33 channels up, 2 from 17, else 1: the network's 32- and 8-channel
-// layers multiplied 2 and 8 times their channels in tiles of 64.
+// layers multiplied 2 and 8 times their channels in tiles of 64.  Measured in a
+// 2 x 384 x 1152, base-32 training step: 32 -> 32 about 110 -> 43 us.
 constexpr int kCPitch = 40;   // LDS row (32 channels of a pixel or weight row) in halves
 
 template <int KS, int NT, bool F32OUT>
@@ -176,7 +177,130 @@ __global__ void __launch_bounds__(256, 2) conv_c32_kernel(const uint16_t *__rest
     }
 }
 
-// More than 32 input channels.  Block: 4 waves, 128 consecutive pixels of one
+// 33 to 32 NC input channels, NC 2 to 4: the same tile with every channel of the
+// block's pixels in LDS at once (rows of 64 NC + 16 bytes: as conflict-free), one
+// block a CU, so that the sum still runs over the taps first and the channels
+// within a tap (an activation rounds to the same bf16).  Measured in that step,
+// operands from L1 before: 64 channels 155 -> 70 us on average, 96 -> 32 at the
+// finest level 266 -> 181 us, 128 channels 50 us.
+template <int KS, int NT, int NC, bool F32OUT>
+__global__ void __launch_bounds__(256)
+conv_lds_kernel(const uint16_t *__restrict__ in, int H, int W, int cin, int is, const uint16_t *__restrict__ w, int cout,
+                const float *__restrict__ bias, int relu, void *__restrict__ out, int os, int ncot, int vec)
+{
+    constexpr int R = KS / 2, IW = 64 + 2 * R, IH = 4 + 2 * R, CO = 16 * NT, PT = 32 * NC + 8;
+    constexpr int NI = IH * IW * 4 * NC, NW = KS * CO * 4 * NC;   // 16-byte units staged
+    constexpr int UW = (NW + 255) / 256;
+    __shared__ __attribute__((aligned(16))) uint16_t sI[IH * IW * PT];
+    __shared__ __attribute__((aligned(16))) uint16_t sW[KS * CO * PT];
+    const int tid = int(threadIdx.x), lane = tid & 63, wv = tid >> 6;
+    const int r16 = lane & 15, g = lane >> 4;
+    const int x0 = int(blockIdx.x) * 64, y0 = int(blockIdx.y) * 4;
+    const int n = int(blockIdx.z) / ncot, co0 = (int(blockIdx.z) % ncot) * CO;
+    f32x4 acc[4][NT];
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    u32x4 rw[UW];
+    auto fetch_w = [&](int dy) {   // the KS taps of row dy
+#pragma unroll
+        for (int u = 0; u < UW; ++u) {
+            const int k = tid + 256 * u, row = k / (4 * NC), ci = k % (4 * NC) * 8;
+            const int dx = row / CO, co = co0 + row % CO;
+            rw[u] = u32x4{0u, 0u, 0u, 0u};
+            if (row < KS * CO && ci < cin && co < cout)
+                rw[u] = *reinterpret_cast<const u32x4 *>(w + (int64_t(co) * (KS * KS) + dy * KS + dx) * cin + ci);
+        }
+    };
+    fetch_w(0);
+    // the pixels and their halo (zeros outside), eight loads in flight a thread
+    // (unrolled whole, the loop was slower: 81, 234 and 55 us for 70, 181 and 50)
+    for (int k0 = tid; k0 < NI; k0 += 256 * 8) {
+        u32x4 ri[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int k = k0 + 256 * u, px = k / (4 * NC), ci = k % (4 * NC) * 8;
+            const int y = y0 - R + px / IW, x = x0 - R + px % IW;
+            ri[u] = u32x4{0u, 0u, 0u, 0u};
+            if (k < NI && ci < cin && y >= 0 && y < H && x >= 0 && x < W)
+                ri[u] = *reinterpret_cast<const u32x4 *>(in + ((int64_t(n) * H + y) * W + x) * is + ci);
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int k = k0 + 256 * u;
+            if (k < NI) *reinterpret_cast<u32x4 *>(sI + k / (4 * NC) * PT + k % (4 * NC) * 8) = ri[u];
+        }
+    }
+#pragma unroll
+    for (int dy = 0; dy < KS; ++dy) {
+        if (dy > 0) __syncthreads();
+#pragma unroll
+        for (int u = 0; u < UW; ++u) {
+            const int k = tid + 256 * u;
+            if (k < NW) *reinterpret_cast<u32x4 *>(sW + k / (4 * NC) * PT + k % (4 * NC) * 8) = rw[u];
+        }
+        __syncthreads();
+        if (dy + 1 < KS) fetch_w(dy + 1);
+#pragma unroll
+        for (int dx = 0; dx < KS; ++dx)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                bf16x8 wf[NT], px[4];
+#pragma unroll
+                for (int t = 0; t < NT; ++t) wf[t] = ld8(sW + (dx * CO + 16 * t + r16) * PT + 32 * c + 8 * g);
+#pragma unroll
+                for (int m = 0; m < 4; ++m)
+                    px[m] = ld8(sI + ((wv + dy) * IW + 16 * m + r16 + dx) * PT + 32 * c + 8 * g);
+#pragma unroll
+                for (int m = 0; m < 4; ++m)
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) acc[m][t] = mma(wf[t], px[m], acc[m][t]);
+            }
+    }
+    const int y = y0 + wv;
+    if (y >= H) return;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int co = co0 + 16 * t + 4 * g;
+        if (co >= cout) continue;
+        float bv[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bv[e] = bias && co + e < cout ? bias[co + e] : 0.f;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            const int x = x0 + 16 * m + r16;
+            if (x >= W) continue;
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[e] = acc[m][t][e] + bv[e];
+                if (relu) v[e] = fmaxf(v[e], 0.f);
+            }
+            const int64_t i = ((int64_t(n) * H + y) * W + x) * os + co;
+            if (vec && co + 4 <= cout) {   // four channels in one store (out and os allow it)
+                if constexpr (F32OUT) {
+                    *reinterpret_cast<f32x4 *>(static_cast<float *>(out) + i) = f32x4{v[0], v[1], v[2], v[3]};
+                } else {
+                    typedef __attribute__((__vector_size__(2 * sizeof(uint32_t)))) uint32_t u32x2;
+                    *reinterpret_cast<u32x2 *>(static_cast<uint16_t *>(out) + i) =
+                        u32x2{uint32_t(f2bf(v[0])) | uint32_t(f2bf(v[1])) << 16,
+                              uint32_t(f2bf(v[2])) | uint32_t(f2bf(v[3])) << 16};
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (co + e >= cout) break;
+                    if constexpr (F32OUT) static_cast<float *>(out)[i + e] = v[e];
+                    else static_cast<uint16_t *>(out)[i + e] = f2bf(v[e]);
+                }
+            }
+        }
+    }
+}
+
+// More than 128 input channels.  Block: 4 waves, 128 consecutive pixels of one
 // image row (32 per wave, two 16-row A tiles) x 16 NT output channels.
 // Grid: (ceil(W / 128), H, N * ceil(cout / (16 NT))).  Every operand comes from
 // L1 or L2; staging a chunk of the input for all taps instead would sum the
@@ -577,6 +701,118 @@ __global__ void __launch_bounds__(256) up2_bwd_kernel(const uint16_t *__restrict
     }
 }
 
+// The same passes on eight channels (16 bytes) a thread, for views whose
+// channels and strides are multiples of 8 on 16-byte aligned pointers, with a
+// 32-bit index.  One channel a thread spent its time on 64-bit divisions and
+// 2-byte accesses: in a 2 x 384 x 1152, base-32 training step relu 25, upsample
+// 106 / 39, pool 22 / 62, column sum 34 us a call.
+__device__ __forceinline__ void unpack8(const u32x4 v, float (&f)[8])
+{
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        f[2 * e] = bf2f(uint16_t(v[e] & 0xffffu));
+        f[2 * e + 1] = bf2f(uint16_t(v[e] >> 16));
+    }
+}
+__device__ __forceinline__ u32x4 pack8(const float (&f)[8])
+{
+    u32x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = uint32_t(f2bf(f[2 * e])) | uint32_t(f2bf(f[2 * e + 1])) << 16;
+    return v;
+}
+__device__ __forceinline__ u32x4 at8(const uint16_t *p, int64_t i) { return *reinterpret_cast<const u32x4 *>(p + i); }
+__device__ __forceinline__ void put8(uint16_t *p, int64_t i, u32x4 v) { *reinterpret_cast<u32x4 *>(p + i) = v; }
+
+__global__ void __launch_bounds__(256) relu_bwd8_kernel(uint16_t *__restrict__ d, int dsd,
+                                                        const uint16_t *__restrict__ act, int as, unsigned n, unsigned C8)
+{
+    for (unsigned i = blockIdx.x * 256u + threadIdx.x; i < n; i += gridDim.x * 256u) {
+        const int64_t p = i / C8;
+        const int c = int(i % C8) * 8;
+        float a[8];
+        unpack8(at8(act, p * as + c), a);
+        u32x4 v = at8(d, p * dsd + c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            v[e] &= (a[2 * e] > 0.f ? 0xffffu : 0u) | (a[2 * e + 1] > 0.f ? 0xffff0000u : 0u);
+        put8(d, p * dsd + c, v);
+    }
+}
+
+// Coarse pixel q of (H, W) per (image): the fine pixel at its corner.
+__device__ __forceinline__ int64_t fine00(unsigned q, int H, int W)
+{
+    const unsigned x = q % unsigned(W), r = q / unsigned(W), y = r % unsigned(H), nn = r / unsigned(H);
+    return (int64_t(nn) * 2 * H + 2 * y) * (2 * int64_t(W)) + 2 * x;
+}
+
+// MODE 0: upsample (coarse -> fine); 1: its adjoint; 2: average pool (fine ->
+// coarse); 3: its adjoint, added into the fine gradient.  H, W: coarse extents.
+template <int MODE>
+__global__ void __launch_bounds__(256) scale2_kernel(uint16_t *__restrict__ coarse, int cs, uint16_t *__restrict__ fine,
+                                                     int fs, int H, int W, unsigned n, unsigned C8)
+{
+    for (unsigned i = blockIdx.x * 256u + threadIdx.x; i < n; i += gridDim.x * 256u) {
+        const unsigned q = i / C8;
+        const int c = int(i % C8) * 8;
+        const int64_t f00 = fine00(q, H, W), W2 = 2 * int64_t(W);
+        const int64_t at[4] = {f00 * fs + c, (f00 + 1) * fs + c, (f00 + W2) * fs + c, (f00 + W2 + 1) * fs + c};
+        const int64_t ac = int64_t(q) * cs + c;
+        if constexpr (MODE == 0) {
+            const u32x4 v = at8(coarse, ac);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) put8(fine, at[k], v);
+        } else if constexpr (MODE == 3) {
+            float d[8];
+            unpack8(at8(coarse, ac), d);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                float f[8];
+                unpack8(at8(fine, at[k]), f);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) f[e] = f[e] + 0.25f * d[e];
+                put8(fine, at[k], pack8(f));
+            }
+        } else {
+            float f[4][8], o[8];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) unpack8(at8(fine, at[k]), f[k]);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float sum = (f[0][e] + f[1][e]) + (f[2][e] + f[3][e]);
+                o[e] = MODE == 2 ? 0.25f * sum : sum;
+            }
+            put8(coarse, ac, pack8(o));
+        }
+    }
+}
+
+// Column sums on eight channels a thread (C a multiple of 8, at most 2048).
+__global__ void __launch_bounds__(256) colsum8_kernel(const uint16_t *__restrict__ x, int xs, int C, int64_t P,
+                                                      int64_t per, float *__restrict__ partial)
+{
+    __shared__ float red[256][9];
+    const int64_t pb = int64_t(blockIdx.x) * per, pe = std::min(P, pb + per);
+    const int C8 = C / 8, J = 256 / C8, t = int(threadIdx.x), j = t / C8, cl = t % C8;
+    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (j < J)
+        for (int64_t p = pb + j; p < pe; p += J) {
+            float f[8];
+            unpack8(at8(x, p * xs + cl * 8), f);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s[e] += f[e];
+        }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) red[t][e] = s[e];
+    __syncthreads();
+    for (int c = t; c < C; c += 256) {
+        float tot = 0.f;
+        for (int k = 0; k < J; ++k) tot += red[k * C8 + c / 8][c % 8];
+        partial[int64_t(blockIdx.x) * C + c] = tot;
+    }
+}
+
 struct Planes {
     const float *p[4];
     float s[4];
@@ -657,6 +893,13 @@ __global__ void __launch_bounds__(256) to_bf16_kernel(const float *__restrict__ 
 
 unsigned blocks_for(int64_t n) { return unsigned(std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 16384))); }
 
+// Whether a pass over n8 groups of 8 channels can run 16 bytes a thread.
+bool vec8(int C, int64_t n8, const void *a, int as, const void *b, int bs)
+{
+    return C % 8 == 0 && as % 8 == 0 && bs % 8 == 0 &&
+           ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0 && n8 < (int64_t(1) << 31);
+}
+
 void check_view(const void *p, int stride, int channels, const char *what)
 {
     SWP_CHECK(p != nullptr, what, ": null pointer");
@@ -705,15 +948,21 @@ void conv_fwd(const uint16_t *in, int N, int H, int W, int cin, int in_stride, c
     const int r = relu ? 1 : 0;
     const int vec = out_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & (out_f32 ? 15 : 7)) == 0;
     const dim3 grid(unsigned((W + 127) / 128), unsigned(H), unsigned(N * ncot));
-    const dim3 grid32(unsigned((W + 63) / 64), unsigned((H + 3) / 4), unsigned(N * ncot));
-#define SWP_CONV_LAUNCH(KS, NT, F32)                                                                               \
-    do {                                                                                                           \
-        if (cin <= 32)                                                                                             \
-            hipLaunchKernelGGL((conv_c32_kernel<KS, NT, F32>), grid32, dim3(256), 0, stream(), in, H, W, cin,      \
-                               in_stride, w, cout, bias, r, out, out_stride, ncot, vec);                           \
-        else                                                                                                       \
-            hipLaunchKernelGGL((conv_fwd_kernel<KS, NT, F32>), grid, dim3(256), 0, stream(), in, H, W, cin,        \
-                               in_stride, w, cout, bias, r, out, out_stride, ncot);                                \
+    const dim3 grid_lds(unsigned((W + 63) / 64), unsigned((H + 3) / 4), unsigned(N * ncot));
+#define SWP_CONV_LDS(KS, NT, NC, F32)                                                                             \
+    hipLaunchKernelGGL((conv_lds_kernel<KS, NT, NC, F32>), grid_lds, dim3(256), 0, stream(), in, H, W, cin,       \
+                       in_stride, w, cout, bias, r, out, out_stride, ncot, vec)
+#define SWP_CONV_LAUNCH(KS, NT, F32)                                                                              \
+    do {                                                                                                          \
+        if (cin <= 32)                                                                                            \
+            hipLaunchKernelGGL((conv_c32_kernel<KS, NT, F32>), grid_lds, dim3(256), 0, stream(), in, H, W, cin,   \
+                               in_stride, w, cout, bias, r, out, out_stride, ncot, vec);                          \
+        else if (cin <= 64) SWP_CONV_LDS(KS, NT, 2, F32);                                                         \
+        else if (cin <= 96) SWP_CONV_LDS(KS, NT, 3, F32);                                                         \
+        else if (cin <= 128) SWP_CONV_LDS(KS, NT, 4, F32);                                                        \
+        else                                                                                                      \
+            hipLaunchKernelGGL((conv_fwd_kernel<KS, NT, F32>), grid, dim3(256), 0, stream(), in, H, W, cin,       \
+                               in_stride, w, cout, bias, r, out, out_stride, ncot);                               \
     } while (0)
 #define SWP_CONV_NT(KS, F32)                         \
     do {                                             \
@@ -729,6 +978,7 @@ void conv_fwd(const uint16_t *in, int N, int H, int W, int cin, int in_stride, c
         else SWP_CONV_NT(1, false);
     }
 #undef SWP_CONV_NT
+#undef SWP_CONV_LDS
 #undef SWP_CONV_LAUNCH
     SWP_LAUNCHED();
 }
@@ -770,8 +1020,12 @@ void conv_wgrad(const uint16_t *in, int N, int H, int W, int cin, int in_stride,
     if (db) {
         float *cp = partials + int64_t(splits) * ks * ks * cout * cin;
         const int64_t cper = (P + kColSplits - 1) / kColSplits;
-        hipLaunchKernelGGL(colsum_kernel, dim3(kColSplits), dim3(256), 0, stream(), dout, dout_stride, cout, P, cper,
-                           cp);
+        if (cout <= 2048)
+            hipLaunchKernelGGL(colsum8_kernel, dim3(kColSplits), dim3(256), 0, stream(), dout, dout_stride, cout, P, cper,
+                               cp);
+        else
+            hipLaunchKernelGGL(colsum_kernel, dim3(kColSplits), dim3(256), 0, stream(), dout, dout_stride, cout, P, cper,
+                               cp);
         SWP_LAUNCHED();
         hipLaunchKernelGGL(colsum_reduce_kernel, dim3(unsigned(cout)), dim3(256), 0, stream(), cp, kColSplits, cout,
                            db);
@@ -790,6 +1044,12 @@ void conv_flip(const uint16_t *w, int cout, int cin, int ks, uint16_t *wt)
 void relu_bwd(uint16_t *d, int d_stride, const uint16_t *act, int act_stride, int64_t P, int C)
 {
     SWP_CHECK(d && act && C >= 1 && C <= d_stride && C <= act_stride, "relu_bwd: bad views");
+    if (vec8(C, P * C / 8, d, d_stride, act, act_stride)) {
+        hipLaunchKernelGGL(relu_bwd8_kernel, dim3(blocks_for(P * C / 8)), dim3(256), 0, stream(), d, d_stride, act,
+                           act_stride, unsigned(P * C / 8), unsigned(C / 8));
+        SWP_LAUNCHED();
+        return;
+    }
     hipLaunchKernelGGL(relu_bwd_kernel, dim3(blocks_for(P * C)), dim3(256), 0, stream(), d, d_stride, act,
                        act_stride, P, C);
     SWP_LAUNCHED();
@@ -799,6 +1059,12 @@ void pool2_fwd(const uint16_t *in, int in_stride, int N, int H, int W, int C, ui
 {
     SWP_CHECK(H % 2 == 0 && W % 2 == 0, "pool2: extents must be even");
     SWP_CHECK(in && out && C <= in_stride && C <= out_stride, "pool2: bad views");
+    if (const int64_t n8 = int64_t(N) * (H / 2) * (W / 2) * (C / 8); vec8(C, n8, out, out_stride, in, in_stride)) {
+        hipLaunchKernelGGL(scale2_kernel<2>, dim3(blocks_for(n8)), dim3(256), 0, stream(), const_cast<uint16_t *>(out),
+                           out_stride, const_cast<uint16_t *>(in), in_stride, H / 2, W / 2, unsigned(n8), unsigned(C / 8));
+        SWP_LAUNCHED();
+        return;
+    }
     hipLaunchKernelGGL(pool2_fwd_kernel, dim3(blocks_for(int64_t(N) * H * W * C / 4)), dim3(256), 0, stream(), in,
                        in_stride, N, H, W, C, out, out_stride);
     SWP_LAUNCHED();
@@ -808,6 +1074,12 @@ void pool2_bwd_acc(const uint16_t *dout, int dout_stride, int N, int H, int W, i
 {
     SWP_CHECK(H % 2 == 0 && W % 2 == 0, "pool2: extents must be even");
     SWP_CHECK(dout && din && C <= dout_stride && C <= din_stride, "pool2: bad views");
+    if (const int64_t n8 = int64_t(N) * (H / 2) * (W / 2) * (C / 8); vec8(C, n8, dout, dout_stride, din, din_stride)) {
+        hipLaunchKernelGGL(scale2_kernel<3>, dim3(blocks_for(n8)), dim3(256), 0, stream(), const_cast<uint16_t *>(dout),
+                           dout_stride, const_cast<uint16_t *>(din), din_stride, H / 2, W / 2, unsigned(n8), unsigned(C / 8));
+        SWP_LAUNCHED();
+        return;
+    }
     hipLaunchKernelGGL(pool2_bwd_kernel, dim3(blocks_for(int64_t(N) * H * W * C)), dim3(256), 0, stream(), dout,
                        dout_stride, N, H, W, C, din, din_stride);
     SWP_LAUNCHED();
@@ -816,6 +1088,12 @@ void pool2_bwd_acc(const uint16_t *dout, int dout_stride, int N, int H, int W, i
 void up2_fwd(const uint16_t *in, int in_stride, int N, int H, int W, int C, uint16_t *out, int out_stride)
 {
     SWP_CHECK(in && out && C <= in_stride && C <= out_stride, "up2: bad views");
+    if (const int64_t n8 = int64_t(N) * H * W * (C / 8); vec8(C, n8, in, in_stride, out, out_stride)) {
+        hipLaunchKernelGGL(scale2_kernel<0>, dim3(blocks_for(n8)), dim3(256), 0, stream(), const_cast<uint16_t *>(in),
+                           in_stride, const_cast<uint16_t *>(out), out_stride, H, W, unsigned(n8), unsigned(C / 8));
+        SWP_LAUNCHED();
+        return;
+    }
     hipLaunchKernelGGL(up2_fwd_kernel, dim3(blocks_for(int64_t(N) * H * W * C * 4)), dim3(256), 0, stream(), in,
                        in_stride, N, H, W, C, out, out_stride);
     SWP_LAUNCHED();
@@ -824,6 +1102,12 @@ void up2_fwd(const uint16_t *in, int in_stride, int N, int H, int W, int C, uint
 void up2_bwd(const uint16_t *dout, int dout_stride, int N, int H, int W, int C, uint16_t *din, int din_stride)
 {
     SWP_CHECK(dout && din && C <= dout_stride && C <= din_stride, "up2: bad views");
+    if (const int64_t n8 = int64_t(N) * H * W * (C / 8); vec8(C, n8, din, din_stride, dout, dout_stride)) {
+        hipLaunchKernelGGL(scale2_kernel<1>, dim3(blocks_for(n8)), dim3(256), 0, stream(), const_cast<uint16_t *>(din),
+                           din_stride, const_cast<uint16_t *>(dout), dout_stride, H, W, unsigned(n8), unsigned(C / 8));
+        SWP_LAUNCHED();
+        return;
+    }
     hipLaunchKernelGGL(up2_bwd_kernel, dim3(blocks_for(int64_t(N) * H * W * C)), dim3(256), 0, stream(), dout,
                        dout_stride, N, H, W, C, din, din_stride);
     SWP_LAUNCHED();
