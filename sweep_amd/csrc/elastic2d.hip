@@ -332,50 +332,49 @@ __global__ void __launch_bounds__(256) stress_prep_kernel(Geo g, Prof pr, Fields
     a.f[M_VXZ][off + i] = pr.azh[iz] * t_vxz;
 }
 
-// stress apply: v_bar += transposed derivatives of q (kernels.cuh:744-832)
+// stress apply, v_bar += transposed derivatives of q on the computed box
+// (kernels.cuh:744-832), and with the cell's own result the velocity prepare of
+// every cell, p = dt / rho v_bar, CPML-filtered (kernels.cuh:870-960).  The
+// prepare reads no neighbour, so it takes v_bar from the registers instead of
+// a pass of its own.
 template <int MS>
-__global__ void __launch_bounds__(256) stress_apply_kernel(Geo g, SCoef c, Fields a, Fields q)
+__global__ void __launch_bounds__(256) stress_apply_kernel(Geo g, SCoef c, Prof pr, Fields a,
+                                                           const float *__restrict__ rhob, Fields q)
 {
     const int M = MS > 0 ? MS : g.M;
-    const int ix = M + int(blockIdx.x) * 64 + int(threadIdx.x);
-    const int iz = M + int(blockIdx.y) * 4 + int(threadIdx.y);
-    const int b = blockIdx.z;
-    if (ix >= g.nx - M || iz >= g.nz - M) return;
-    const int64_t off = int64_t(b) * g.n, i = int64_t(iz) * g.nx + ix, nx = g.nx;
-    const float dqxx_dx = sgd<MS, true>(c, q.f[0] + off, i, 1, g.inv_dx, M);
-    const float dqxz_dz = sgd<MS, false>(c, q.f[2] + off, i, nx, g.inv_dz, M);
-    const float dqzx_dx = sgd<MS, false>(c, q.f[3] + off, i, 1, g.inv_dx, M);
-    const float dqzz_dz = sgd<MS, true>(c, q.f[1] + off, i, nx, g.inv_dz, M);
-    a.f[VX][off + i] += dqxx_dx + dqxz_dz;
-    a.f[VZ][off + i] += dqzx_dx + dqzz_dz;
-}
-
-// velocity prepare (every cell): p = dt / rho v_bar, CPML-filtered (kernels.cuh:870-960)
-__global__ void __launch_bounds__(256) vel_prep_kernel(Geo g, Prof pr, Fields a, const float *__restrict__ rhob, Fields p)
-{
     const int ix = int(blockIdx.x) * 64 + int(threadIdx.x);
     const int iz = int(blockIdx.y) * 4 + int(threadIdx.y);
     const int b = blockIdx.z;
     if (ix >= g.nx || iz >= g.nz) return;
-    const int64_t off = int64_t(b) * g.n, i = int64_t(iz) * g.nx + ix;
+    const int64_t off = int64_t(b) * g.n, i = int64_t(iz) * g.nx + ix, nx = g.nx;
+    float vx = a.f[VX][off + i], vz = a.f[VZ][off + i];
+    if (ix >= M && ix < g.nx - M && iz >= M && iz < g.nz - M) {
+        const float dqxx_dx = sgd<MS, true>(c, q.f[0] + off, i, 1, g.inv_dx, M);
+        const float dqxz_dz = sgd<MS, false>(c, q.f[2] + off, i, nx, g.inv_dz, M);
+        const float dqzx_dx = sgd<MS, false>(c, q.f[3] + off, i, 1, g.inv_dx, M);
+        const float dqzz_dz = sgd<MS, true>(c, q.f[1] + off, i, nx, g.inv_dz, M);
+        vx += dqxx_dx + dqxz_dz;
+        vz += dqzx_dx + dqzz_dz;
+        a.f[VX][off + i] = vx;
+        a.f[VZ][off + i] = vz;
+    }
     const float inv_rho = 1.f / rhob[int64_t(b) * g.mstride + i];
-    const float vx = a.f[VX][off + i], vz = a.f[VZ][off + i];
     const float bar_dsxx_dx = g.dt * inv_rho * vx, bar_dsxz_dz = g.dt * inv_rho * vx;
     const float bar_dsxz_dx = g.dt * inv_rho * vz, bar_dszz_dz = g.dt * inv_rho * vz;
-    // p.f[4..7] = pxx, pzz, pxz, pzx
+    // q.f[4..7] = pxx, pzz, pxz, pzx
     if (!in_pml(g, ix, iz)) {
-        p.f[4][off + i] = bar_dsxx_dx;
-        p.f[6][off + i] = bar_dsxz_dz;
-        p.f[7][off + i] = bar_dsxz_dx;
-        p.f[5][off + i] = bar_dszz_dz;
+        q.f[4][off + i] = bar_dsxx_dx;
+        q.f[6][off + i] = bar_dsxz_dz;
+        q.f[7][off + i] = bar_dsxz_dx;
+        q.f[5][off + i] = bar_dszz_dz;
         return;
     }
     const float t_sxxx = a.f[M_SXXX][off + i] + bar_dsxx_dx, t_sxzz = a.f[M_SXZZ][off + i] + bar_dsxz_dz;
     const float t_sxzx = a.f[M_SXZX][off + i] + bar_dsxz_dx, t_szzz = a.f[M_SZZZ][off + i] + bar_dszz_dz;
-    p.f[4][off + i] = bar_dsxx_dx + pr.bxh[ix] * t_sxxx;
-    p.f[6][off + i] = bar_dsxz_dz + pr.bz[iz] * t_sxzz;
-    p.f[7][off + i] = bar_dsxz_dx + pr.bx[ix] * t_sxzx;
-    p.f[5][off + i] = bar_dszz_dz + pr.bzh[iz] * t_szzz;
+    q.f[4][off + i] = bar_dsxx_dx + pr.bxh[ix] * t_sxxx;
+    q.f[6][off + i] = bar_dsxz_dz + pr.bz[iz] * t_sxzz;
+    q.f[7][off + i] = bar_dsxz_dx + pr.bx[ix] * t_sxzx;
+    q.f[5][off + i] = bar_dszz_dz + pr.bzh[iz] * t_szzz;
     a.f[M_SXXX][off + i] = pr.axh[ix] * t_sxxx;
     a.f[M_SXZX][off + i] = pr.ax[ix] * t_sxzx;
     a.f[M_SXZZ][off + i] = pr.az[iz] * t_sxzz;
@@ -742,8 +741,7 @@ void reverse_step(const Ctx &x, const swp_problem &p, const swp_backward_io &io,
         by_order(g.M, [&](auto ms) {
             constexpr int MS = decltype(ms)::value;
             hipLaunchKernelGGL(stress_prep_kernel, all, dim3(64, 4), 0, stream(), g, x.pr, w.a, w.md.lam, w.md.mu, w.qp);
-            hipLaunchKernelGGL(stress_apply_kernel<MS>, in, dim3(64, 4), 0, stream(), g, x.c, w.a, w.qp);
-            hipLaunchKernelGGL(vel_prep_kernel, all, dim3(64, 4), 0, stream(), g, x.pr, w.a, p.models[2], w.qp);
+            hipLaunchKernelGGL(stress_apply_kernel<MS>, all, dim3(64, 4), 0, stream(), g, x.c, x.pr, w.a, p.models[2], w.qp);
             hipLaunchKernelGGL(vel_apply_kernel<MS>, in, dim3(64, 4), 0, stream(), g, x.c, w.a, w.qp);
         });
         SWP_LAUNCHED();
