@@ -733,7 +733,7 @@ void forward(const Ctx &x, const swp_problem &p_in, float *record)
 // One adjoint step: stencil, residual injection at the receivers, rotation,
 // then the wavelet-gradient gather at the sources (eq_driver.cuh:689-698).
 static void adjoint_step(const Ctx &x, const swp_problem &p, const swp_backward_io &io,
-                         AdjState &a, int it, const float *img, float *grad)
+                         AdjState &a, int it, const float *img, float *grad, const PointArgs *also = nullptr)
 {
     const Geo &g = x.g;
     AdjFields f{p.models[0], a.l[0], a.l[1], a.l[2], a.psix, a.psiz, a.zetax, a.zetaz,
@@ -754,7 +754,12 @@ static void adjoint_step(const Ctx &x, const swp_problem &p, const swp_backward_
     }
     {
         TimedScope ts(K_OTHER);
-        launch_points(pa, g.B);
+        if (also) {
+            const PointArgs both[2] = {pa, *also};
+            launch_points(both, 2, g.B);
+        } else {
+            launch_points(pa, g.B);
+        }
     }
     float *t = a.l[0];
     a.l[0] = a.l[1];
@@ -888,8 +893,11 @@ static void backward_run(const Ctx &x, const swp_problem &p, const swp_backward_
     }
     const int bw = g.X1 - g.X0, bh = g.Z1 - g.Z0 - wzl - wzh;
     const int n_strip = (wzl + wzh) * bw + (wxl + wxh) * std::max(bh, 0);
+    // The source goes back into a reconstructed field only before the next
+    // reconstruction reads it, so it rides on the next step's residual pass.
+    PointArgs back = point_args(g);
     for (int it = g.nt - 1; it >= 1; --it) {
-        adjoint_step(x, p, io, a, it, nullptr, nullptr);
+        adjoint_step(x, p, io, a, it, nullptr, nullptr, it + 1 < g.nt ? &back : nullptr);
         const float *lam = a.l[1];
         if (bxl < g.nx - bxh && bzl < g.nz - bzh) {
             TimedScope ts(K_RECON);
@@ -915,16 +923,11 @@ static void backward_run(const Ctx &x, const swp_problem &p, const swp_backward_
             SWP_LAUNCHED();
         }
         if (S || R) image(x, p, r[0], r[2], r[1], lam, nullptr, S, R);
-        PointArgs pa = point_args(g);
-        pa.it = it;
-        pa.u_add = r[2];
-        pa.add_w = p.source;
-        pa.add_loc = p.sources_loc;
-        pa.nadd = p.nsrc;
-        {
-            TimedScope ts(K_OTHER);
-            launch_points(pa, g.B);
-        }
+        back.it = it;
+        back.u_add = r[2];
+        back.add_w = p.source;
+        back.add_loc = p.sources_loc;
+        back.nadd = p.nsrc;
         float *tp = r[0];
         r[0] = r[1];
         r[1] = r[2];

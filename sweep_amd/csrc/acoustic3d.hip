@@ -717,7 +717,7 @@ void forward(const swp_problem &p_in, float *record)
 }
 
 static void adjoint_step(const Ctx &x, const swp_problem &p, const swp_backward_io &io, AdjState &a, int it,
-                         const float *img, float *grad)
+                         const float *img, float *grad, const PointArgs *also = nullptr)
 {
     const Geo &g = x.g;
     AdjFields f{};
@@ -747,7 +747,12 @@ static void adjoint_step(const Ctx &x, const swp_problem &p, const swp_backward_
     }
     {
         TimedScope ts(K_OTHER);
-        launch_points(pa, g.B);
+        if (also) {
+            const PointArgs both[2] = {pa, *also};
+            launch_points(both, 2, g.B);
+        } else {
+            launch_points(pa, g.B);
+        }
     }
     float *t = a.l[0];
     a.l[0] = a.l[1];
@@ -890,8 +895,11 @@ static void backward_run(const Ctx &x, const swp_problem &p, const swp_backward_
     const int64_t mz = std::max(g.nzp - sw.zl - sw.zh, 0), my = std::max(g.nyp - sw.yl - sw.yh, 0);
     const int64_t n_strip = int64_t(sw.zl + sw.zh) * g.nyp * g.nxp + mz * (sw.yl + sw.yh) * g.nxp +
                             mz * my * (sw.xl + sw.xh);
+    // The source goes back into a reconstructed field only before the next
+    // reconstruction reads it, so it rides on the next step's residual pass.
+    PointArgs back = point_args(g);
     for (int it = g.nt - 1; it >= 1; --it) {
-        adjoint_step(x, p, io, a, it, nullptr, nullptr);
+        adjoint_step(x, p, io, a, it, nullptr, nullptr, it + 1 < g.nt ? &back : nullptr);
         const float *lam = a.l[1];
         if (recon) launch_recon(x, p.models[0], r[0], r[1], r[2], lam, grad, bx);
         if (n_strip > 0) {
@@ -902,16 +910,11 @@ static void backward_run(const Ctx &x, const swp_problem &p, const swp_backward_
             SWP_LAUNCHED();
         }
         if (S || R) image(x, p, r[0], r[2], r[1], lam, nullptr, S, R);
-        PointArgs pa = point_args(g);
-        pa.it = it;
-        pa.u_add = r[2];
-        pa.add_w = p.source;
-        pa.add_loc = p.sources_loc;
-        pa.nadd = p.nsrc;
-        {
-            TimedScope ts(K_OTHER);
-            launch_points(pa, g.B);
-        }
+        back.it = it;
+        back.u_add = r[2];
+        back.add_w = p.source;
+        back.add_loc = p.sources_loc;
+        back.nadd = p.nsrc;
         float *tp = r[0];
         r[0] = r[1];
         r[1] = r[2];

@@ -27,6 +27,11 @@ struct PointArgs {
 
 void launch_points(const PointArgs &a, int B);
 
+// n independent passes, two a launch: no field is in two of them.  On a small
+// grid a pass costs its launch (2.5 to 5 us, a sixth of a step of 96 x 128).
+constexpr int kMaxPointPasses = 10;
+void launch_points(const PointArgs *a, int n, int B);
+
 // Boundary strips hold fp32 or, with SWP_FLAG_BF16_STRIPS, bfloat16: round
 // to nearest, ties to even, a NaN kept a quiet NaN (the rounding of the
 // reference's __float2bfloat16).  A strip pointer is typed float* either way;

@@ -631,6 +631,32 @@ PointArgs point_args(const Geo &g)
     return a;
 }
 
+// The passes in one launch where no two of them share a field, else in order
+// (a caller may list a field twice).
+template <class F>
+void launch_fields(const Ctx &x, const PointArgs *pass, int n, F &&field)
+{
+    bool apart = n <= kMaxPointPasses;
+    for (int i = 0; i < n; ++i)
+        for (int j = 0; j < i; ++j) apart = apart && field(i) != field(j);
+    if (apart) {
+        launch_points(pass, n, x.g.B);
+        return;
+    }
+    for (int k = 0; k < n; ++k)   // every source before any record
+        if (pass[k].u_add) {
+            PointArgs a = pass[k];
+            a.u_get = nullptr;
+            launch_points(a, x.g.B);
+        }
+    for (int k = 0; k < n; ++k)
+        if (pass[k].u_get) {
+            PointArgs a = pass[k];
+            a.u_add = nullptr;
+            launch_points(a, x.g.B);
+        }
+}
+
 // One forward step: velocity, stress (capturing v when vcap), sources, records.
 void forward_step(const Ctx &x, const swp_problem &p, Work &w, int it, float *vcap, float *record)
 {
@@ -647,26 +673,35 @@ void forward_step(const Ctx &x, const swp_problem &p, Work &w, int it, float *vc
         SWP_LAUNCHED();
     }
     TimedScope ts(K_OTHER);
-    for (int k = 0; k < x.nsf; ++k) {
-        PointArgs a = point_args(g);
-        a.it = it;
+    // each record field's pass also adds the sources of that field; the other
+    // source fields take passes of their own
+    PointArgs pass[10];
+    int n = 0;
+    bool added[5] = {false, false, false, false, false};
+    auto add_source = [&](PointArgs &a, int k) {
         a.u_add = w.s.f[x.sf[k]];
         a.add_w = p.source;
         a.add_loc = p.sources_loc;
         a.nadd = p.nsrc;
-        launch_points(a, g.B);
+        added[k] = true;
+    };
+    for (int k = 0; record && k < x.nrf; ++k) {
+        PointArgs &a = pass[n++] = point_args(g);
+        a.it = it;
+        a.u_get = w.s.f[x.rf[k]];
+        a.get_out = record + int64_t(k) * g.B * p.nrec * g.nt;
+        a.get_loc = p.receivers_loc;
+        a.nget = p.nrec;
+        for (int j = 0; j < x.nsf; ++j)
+            if (x.sf[j] == x.rf[k] && !added[j] && !a.u_add) add_source(a, j);
     }
-    if (record) {
-        for (int k = 0; k < x.nrf; ++k) {
-            PointArgs a = point_args(g);
-            a.it = it;
-            a.u_get = w.s.f[x.rf[k]];
-            a.get_out = record + int64_t(k) * g.B * p.nrec * g.nt;
-            a.get_loc = p.receivers_loc;
-            a.nget = p.nrec;
-            launch_points(a, g.B);
-        }
+    for (int j = 0; j < x.nsf; ++j) {
+        if (added[j]) continue;
+        PointArgs &a = pass[n++] = point_args(g);
+        a.it = it;
+        add_source(a, j);
     }
+    launch_fields(x, pass, n, [&](int k) { return static_cast<const float *>(pass[k].u_add ? pass[k].u_add : pass[k].u_get); });
 }
 
 void zero_state(const Geo &g, Fields &f)
@@ -713,16 +748,17 @@ void reverse_step(const Ctx &x, const swp_problem &p, const swp_backward_io &io,
             hipLaunchKernelGGL(rho_src_kernel, dim3(unsigned((p.nsrc + 255) / 256), unsigned(g.B)), dim3(256), 0,
                                stream(), g, grho, w.a.f[x.sf[k]], p.models[2], p.source, p.sources_loc, p.nsrc, it);
         }
+        PointArgs pass[5];
         for (int k = 0; k < x.nrf; ++k) {
-            PointArgs a = point_args(g);
+            PointArgs &a = pass[k] = point_args(g);
             a.it = it;
             a.u_add = w.a.f[x.rf[k]];
             a.add_w = io.adjoint_source + int64_t(k) * g.B * p.nrec * g.nt;
             a.add_loc = p.receivers_loc;
             a.nadd = p.nrec;
             a.sign = x.rf[k] >= 2 ? -1.f : 1.f;
-            launch_points(a, g.B);
         }
+        launch_fields(x, pass, x.nrf, [&](int k) { return static_cast<const float *>(pass[k].u_add); });
         SWP_LAUNCHED();
     }
     if constexpr (!std::is_same_v<Between, std::nullptr_t>) between();
