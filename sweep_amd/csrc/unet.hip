@@ -893,11 +893,13 @@ __global__ void __launch_bounds__(256) to_bf16_kernel(const float *__restrict__ 
 
 unsigned blocks_for(int64_t n) { return unsigned(std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 16384))); }
 
-// Whether a pass over n8 groups of 8 channels can run 16 bytes a thread.
+// Whether a pass over n8 groups of 8 channels can run 16 bytes a thread.  The
+// kernels count in 32 bits unsigned; a negative extent stays with the 64-bit
+// passes, which do nothing for it.
 bool vec8(int C, int64_t n8, const void *a, int as, const void *b, int bs)
 {
     return C % 8 == 0 && as % 8 == 0 && bs % 8 == 0 &&
-           ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0 && n8 < (int64_t(1) << 31);
+           ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0 && n8 >= 0 && n8 < (int64_t(1) << 31);
 }
 
 void check_view(const void *p, int stride, int channels, const char *what)

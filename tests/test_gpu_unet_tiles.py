@@ -83,3 +83,19 @@ def test_elementwise_passes_without_groups_of_eight():
     dg = d.to(dev)
     _call("swp_nn_relu_bwd", _p(dg), C, _p(xg), C, N * H * W, C)
     assert torch.equal(dg.cpu(), torch.where(v > 0, d, torch.zeros_like(d)))
+
+
+def test_negative_counts_are_empty():
+    """A negative pixel or image count is an empty range, also for views that
+    the eight-channel passes take."""
+    dev = torch.device("cuda:0")
+    H, W, C = 4, 4, 16
+    a = torch.randn((1, H, W, C), device=dev).to(torch.bfloat16)
+    b = torch.randn((1, 2 * H, 2 * W, C), device=dev).to(torch.bfloat16)
+    a0, b0 = a.clone(), b.clone()
+    _call("swp_nn_relu_bwd", _p(a), C, _p(b), C, -H * W, C)
+    _call("swp_nn_pool2_fwd", _p(b), C, -1, 2 * H, 2 * W, C, _p(a), C)
+    _call("swp_nn_pool2_bwd_acc", _p(a), C, -1, 2 * H, 2 * W, C, _p(b), C)
+    _call("swp_nn_up2_fwd", _p(a), C, -1, H, W, C, _p(b), C)
+    _call("swp_nn_up2_bwd", _p(b), C, -1, H, W, C, _p(a), C)
+    assert torch.equal(a, a0) and torch.equal(b, b0)
