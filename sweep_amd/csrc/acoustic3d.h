@@ -64,7 +64,8 @@ struct Ctx {
     Geo g;
     Coef c;
     Prof pr;
-    bool zm;             // z-marching kernels (fixed orders 2..8)
+    bool zm_fwd;         // forward steps on the z-marching kernels (fixed orders 2..8)
+    bool zm;             // adjoint steps and reconstructions on them
     bool zm_forced;      // the family was forced to z-march (SWP_KERNELS)
     bool big;            // kBigCells3 shot-cells and up: the forward's roundings of that range
     bool shell_percell;  // with zm: the CPML shell on the per-cell kernels

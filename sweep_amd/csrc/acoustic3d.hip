@@ -414,10 +414,10 @@ static void launch_fwd(const Ctx &x, const StepFields &f, float *u_this, float *
 {
     TimedScope ts(K_FWD);
     const Geo &g = x.g;
-    if (x.zm) launch_fwd_zm(x, f, u_this, strip, !x.shell_percell);
-    if (x.zm && !x.shell_percell) return;
+    if (x.zm_fwd) launch_fwd_zm(x, f, u_this, strip, !x.shell_percell);
+    if (x.zm_fwd && !x.shell_percell) return;
     by_order(g.M, [&](auto ms) {
-        per_box(g, x.zm, [&](const Box &bx, dim3 grid) {
+        per_box(g, x.zm_fwd, [&](const Box &bx, dim3 grid) {
             census_add("a3d.fwd_cell", int64_t(grid.x) * grid.y * grid.z);
             hipLaunchKernelGGL(fwd_kernel<decltype(ms)::value>, grid, dim3(64, 4), 0, stream(), g, x.c, x.pr, f,
                                u_this, strip, bx);
@@ -926,6 +926,42 @@ static void backward_run(const Ctx &x, const swp_problem &p, const swp_backward_
     }
 }
 
+// Which family is faster for the forward step and for the adjoint (with the
+// reconstruction) of a launch of kZmMinCells3 to kBigCells3 shot-cells.  The
+// per-cell kernels' loads a cell grow with the order; the march pays its masked
+// lanes (zm_lane_ratio), a barrier a plane and, with few tiles, a last round
+// that is nearly empty.  Time per-cell over z-march, 130 sizes (24..160 x
+// 24..256 x 24..256, one and two shots), by lane ratio and shot-cells:
+//              forward                                      adjoint
+//   order 2  < 1.2 to 10M  1.00..1.17 (0.95..0.98 4 times)  < 1.33  1.03..1.26
+//            to 14M        1.01..1.11 (0.88..0.96 4 times)  >= 1.33 0.88..1.04
+//            above         0.84..1.09
+//            >= 1.33       0.80..0.98
+//   order 4  < 1.33        0.94..1.24 (60^3 0.90)           < 1.4   1.12..1.52
+//            >= 1.33       0.76..1.01 (1.08 once)           >= 1.4  0.91..0.93 to 5M, 1.02..1.21 above
+//   order 6  < 1.4         0.96..1.50                       all     1.05..1.63 (0.96..0.99 thrice)
+//            >= 1.4 to 6M  0.86..0.95, above 1.00..1.15
+//   order 8  < 1.4         1.00..1.64                       all     1.06..1.84
+//            >= 1.4 to 6M  0.90..0.98, above 1.06..1.26
+// Between 1.2 and 1.33 orders 2 and 4 lose up to 5M (0.85..0.98) and gain above.
+// Microseconds a forward step, per-cell / z-march: order 8, 83 x 28 x 85, 72 /
+// 79; order 2, 80 x 80 x 80, 83 / 93; order 4, 97 x 110 x 131, 168 / 143.
+static bool march_fwd(const Geo &g, int64_t cells)
+{
+    if (cells < kZmMinCells3 || cells >= kBigCells3) return cells >= kBigCells3;
+    if (g.M >= 3) return cells >= (int64_t(6) << 20) || zm_lane_ratio(g) < 1.4;
+    if (g.M == 1 && cells >= (int64_t(14) << 20)) return false;
+    return zm_lane_ratio(g) < (cells < (int64_t(5) << 20) ? 1.2 : 1.33);
+}
+
+static bool march_adj(const Geo &g, int64_t cells)
+{
+    if (cells < kZmMinCells3 || cells >= kBigCells3) return cells >= kBigCells3;
+    if (g.M >= 3) return true;
+    if (g.M == 2) return cells >= (int64_t(5) << 20) || zm_lane_ratio(g) < 1.4;
+    return zm_lane_ratio(g) < 1.33;
+}
+
 Ctx make_ctx(const swp_problem &p)
 {
     SWP_CHECK(p.ndim == 3, "acoustic3d: ndim must be 3, got ", p.ndim);
@@ -946,9 +982,9 @@ Ctx make_ctx(const swp_problem &p)
         x.pr.db[a] = p.pml[3 * src + 2];
     }
     x.tz = tuning(SWP_TUNE_TZ3, "SWP_TZ3", 64);
-    // Kernel family, as in 2-D: the z-marching kernels from kZmMinCells3
-    // shot-cells (B x nz x ny x nx on the runtime grid) up, one thread per
-    // cell below, where a launch holds too few z segments.
+    // Kernel family of the forward steps and of the adjoint ones, which read
+    // and write the same layouts: by shot-cells (B x nz x ny x nx on the
+    // runtime grid), order and shape.
     // SWP_KERNELS=percell / zmarch forces a family (zmarch_big: with the
     // roundings of kBigCells3 shot-cells and up).
     const char *kern = std::getenv("SWP_KERNELS");
@@ -956,7 +992,9 @@ Ctx make_ctx(const swp_problem &p)
     const int64_t cells = int64_t(x.g.B) * x.g.nz * x.g.ny * x.g.nx;
     x.big = cells >= kBigCells3 || ks == "zmarch_big";
     x.zm_forced = ks == "zmarch" || ks == "zmarch_big";
-    x.zm = zm_supported(x.g, x.tz) && ks != "percell" && (ks == "zmarch" || ks == "zmarch_big" || cells >= kZmMinCells3);
+    const bool can = zm_supported(x.g, x.tz) && ks != "percell";
+    x.zm_fwd = can && (x.zm_forced || march_fwd(x.g, cells));
+    x.zm = can && (x.zm_forced || march_adj(x.g, cells));
     // SWP_SHELL3=percell runs the CPML shell with the per-cell kernels over
     // six slabs instead of the region-specialised z-marching kernels.
     const char *sh = std::getenv("SWP_SHELL3");

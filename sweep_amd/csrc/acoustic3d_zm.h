@@ -7,9 +7,9 @@ namespace swp {
 namespace a3d {
 
 // Smallest launch (shots x runtime-grid cells) that runs on the z-marching
-// kernels by default; smaller ones run one thread per cell.  Measured per step
-// of forward + adjoint + reconstruction, order 8 (per-cell / z-march): 3.1M
-// shot-cells 164 / 164 us, 6.2M 394 / 310, 9.7M 571 / 425, 12.5M 686 / 452.
+// kernels by default; smaller ones run one thread per cell.  From here to
+// kBigCells3 shot-cells the choice goes by order and shape (march_fwd and
+// march_adj in acoustic3d.hip).
 constexpr int64_t kZmMinCells3 = int64_t(4) << 20;
 // From here up the forward step adds the last axes' second derivatives to the
 // CPML sum in one rounding each; below, every term is rounded first, as the
@@ -23,9 +23,14 @@ constexpr int64_t kBigCells3 = int64_t(32) << 20;
 // times are within 1.5%).
 constexpr int64_t kZmMinRecon3 = int64_t(4) << 20;
 
+// The cells that the z-march's tiles cover, masked lanes included, over those
+// that the per-cell kernels' 64 x 4 blocks cover.  It is near 1 where each x
+// range fills its 64-column tiles, and 1.33 to 1.6 where the middle range of a
+// narrow grid takes a tile more for a few columns.
+double zm_lane_ratio(const Geo &g);
+
 // Orders 2..8, and a z segment of tz planes plus its 2M + 1 halo and prefetch
 // planes addressable with 32-bit byte offsets (tz is clamped to fit).
-
 bool zm_supported(const Geo &g, int &tz);
 // The slabs of the computed box around the lean interior [lo + M + 1,
 // hi - M - 1) per axis (the whole box when that interior is empty); returns

@@ -1280,6 +1280,18 @@ bool zm_supported(const Geo &g, int &tz)
     return true;
 }
 
+double zm_lane_ratio(const Geo &g)
+{
+    int64_t lanes = 0;
+    for (int t = 0; t < 8; ++t) {
+        const int TY = 4 * ry_of(t);
+        const ZSet s = region_set(g, t & 1, t & 2, t & 4, g.nz, TY);
+        for (int j = 0; j < s.n; ++j) lanes += int64_t(64) * s.r[j].ntx * TY * s.r[j].nty * (s.r[j].z1 - s.r[j].z0);
+    }
+    const int64_t cols = int64_t(g.nx - 2 * g.M + 63) / 64 * 64, rows = int64_t(g.ny - 2 * g.M + 3) / 4 * 4;
+    return double(lanes) / double(cols * rows * (g.nz - 2 * g.M));
+}
+
 int shell_boxes(const Geo &g, Box out[6])
 {
     // the six slabs around the lean interior (per-cell shell launches)
