@@ -1232,21 +1232,25 @@ void census_region(const char *what, int type, int64_t blocks)
     census_add(site, blocks);
 }
 
-// Segment height of a launch: tz, halved (down to kMinTz planes) while the
-// launch would have fewer than kMinWaves waves (SWP_REGION_WAVES overrides, 1
-// keeps tz).  A workgroup walks its segment one plane (one load latency) at a
-// time, so a launch of few workgroups takes about tz plane latencies however
-// few cells it holds; a shorter segment repeats its 2M + 1 plane prologue more
-// often.  Measured per gradient at 40 x 36 x 44 (two shots, order 4), 97 x 110
+// Whether a launch takes z segments of half the height: while it would have
+// fewer than kMinWaves waves (SWP_REGION_WAVES overrides, 1 keeps tz) and half
+// of tz is still kMinTz planes or more.  A workgroup walks its segment one plane
+// (one load latency) at a time, so a launch of few workgroups takes about tz
+// plane latencies however few cells it holds; a shorter segment repeats its
+// 2M + 1 plane prologue more often.  Measured per gradient at 40 x 36 x 44 (two shots, order 4), 97 x 110
 // x 131 and, records only, 128 x 256 x 256 (order 8): 8 planes / 16384 waves
 // 41.5, 41.8 and 35.7 ms; 16 planes / 8192 waves 43.7, 44.6 and 36.2 ms.
 constexpr int64_t kMinWaves = 16384;
 constexpr int kMinTz = 8;
 
+bool halve_tz(int tz, int64_t waves)
+{
+    return tz / 2 >= kMinTz && waves < tuning(-1, "SWP_REGION_WAVES", kMinWaves);
+}
+
 // The plan of the region types in `mask` (bit t: type t).
 ZPlan make_zplan(const Geo &g, unsigned mask, int tz)
 {
-    const int64_t min_waves = tuning(-1, "SWP_REGION_WAVES", kMinWaves);
     for (;; tz /= 2) {
         ZPlan p{};
         int64_t blocks = 0;
@@ -1264,7 +1268,7 @@ ZPlan make_zplan(const Geo &g, unsigned mask, int tz)
             SWP_CHECK(blocks < (int64_t(1) << 31), "acoustic3d: launch too large");
             p.first[k + 1] = int(blocks);
         }
-        if (tz <= kMinTz || blocks * 4 >= min_waves) return p;
+        if (!halve_tz(tz, blocks * 4)) return p;
     }
 }
 
@@ -1338,15 +1342,13 @@ void launch_recon_zm(const Ctx &x, const float *vp, const float *u_prev, const f
                      const float *adj, float *grad, int x0, int x1, int y0, int y1, int z0, int z1)
 {
     const Geo &g = x.g;
-    const int64_t min_waves = tuning(-1, "SWP_REGION_WAVES", kMinWaves);
     ZSet s;
-    int tz = x.tz;
-    do {
+    for (int tz = x.tz;; tz /= 2) {
         s = ZSet{};
         add_rect(s, x0, x1, y0, y1, z0, z1, tz, kNwRecon * kRyRecon, x.g.px);
         if (!s.per_shot) return;
-        tz /= 2;
-    } while (tz >= kMinTz && int64_t(s.per_shot) * g.B * kNwRecon < min_waves);
+        if (!halve_tz(tz, int64_t(s.per_shot) * g.B * kNwRecon)) break;
+    }
     census_add("a3d.recon_zm", int64_t(s.per_shot) * g.B);
     by_order(g.M, [&](auto ms) {
         constexpr int M = decltype(ms)::value;

@@ -83,3 +83,32 @@ def test_record_bits_do_not_depend_on_the_family(order, monkeypatch):
         with torch.no_grad():
             out[family] = solver(wav, src, rec, models=[vp])
     assert torch.equal(out["percell"], out["zmarch"])
+
+
+@pytest.mark.parametrize("tz,least", [(64, 8), (48, 12), (9, 9), (5, 5)])
+def test_segments_are_not_halved_below_eight_planes(tz, least, monkeypatch):
+    """A launch of few waves halves its segment height while 8 planes or more
+    remain: it starts as many workgroups as with that height kept."""
+    from sweep_amd import _core
+    from sweep_amd.equations import Acoustic3D
+    from sweep_amd.propagator import PropTorch
+    dev = _dev()
+    monkeypatch.setenv("SWP_KERNELS", "zmarch")
+    vp = torch.full((40, 30, 70), 2000.0, device=dev)
+    wav = np.ones(3, np.float32)
+
+    def census(height, waves):
+        monkeypatch.setenv("SWP_TZ3", str(height))
+        monkeypatch.setenv("SWP_REGION_WAVES", str(waves))
+        solver = PropTorch(Acoustic3D(spatial_order=4, device=dev), shape=vp.shape, dh=9.0, dt=9e-4, device=dev, abcn=8)
+        m = vp.clone().requires_grad_(True)
+        _core.census_enable(True)
+        solver(wav, np.array([[5, 6, 2]]), np.array([[[8, 6, 2]]]), models=[m]).sum().backward()
+        torch.cuda.synchronize()
+        out = {k: v for k, v in _core.census().items() if "3." in k[4:] or k == "a3d.recon_zm"}
+        _core.census_enable(False)
+        return out
+
+    got = census(tz, 1 << 30)
+    assert len(got) > 2
+    assert got == census(least, 1)
