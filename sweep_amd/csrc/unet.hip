@@ -369,8 +369,9 @@ __global__ void __launch_bounds__(256) conv_fwd_kernel(const uint16_t *__restric
 }
 
 // ---------------------------------------------------------------- weight gradient
-// Block: 4 waves, 32 TO output x 32 TI input channels, every tap, over a strip
-// of SP columns and a segment of rows of one image.  The contraction runs over
+// Block: 4 waves, 32 TO output x 32 TI input channels, every tap, over strips
+// of SP columns and a segment of rows of an image: one strip, or several in turn
+// where there are more of them than workgroups (wgrad_plan).  The contraction runs over
 // pixels: each image row of the strip (input with its ks / 2 halo columns, dout
 // without) is staged once in LDS as [pixel][channel] and feeds all ks * ks taps
 // (the input rows of a window stay in a ring), where ds_read_b64_tr_b16 hands a
@@ -416,7 +417,8 @@ __device__ __forceinline__ bf16x8 ld_tr(const uint16_t *p, int pitch)
 template <int KS, int TO, int TI>
 __global__ void __launch_bounds__(256, 2) wgrad_kernel(const uint16_t *__restrict__ in, int H, int W, int cin, int is,
                                                        const uint16_t *__restrict__ dout, int cout, int ds,
-                                                       float *__restrict__ partials, int nsx, int nsy, int rows)
+                                                       float *__restrict__ partials, int nsx, int nsy, int rows,
+                                                       int strips)
 {
     using T = WgradTile<KS, TO, TI>;
     __shared__ __attribute__((aligned(16))) uint16_t mem[T::NS * T::IW * T::PI + 2 * T::SP * T::PD];
@@ -425,8 +427,6 @@ __global__ void __launch_bounds__(256, 2) wgrad_kernel(const uint16_t *__restric
     const int tid = int(threadIdx.x), lane = tid & 63, wv = tid >> 6;
     const int g = lane >> 4, i16 = lane & 15;
     const int ci0 = int(blockIdx.y) * 32 * TI, co0 = int(blockIdx.z) * 32 * TO;
-    const int sx = int(blockIdx.x) % nsx, sy = int(blockIdx.x) / nsx % nsy, n = int(blockIdx.x) / (nsx * nsy);
-    const int x0 = sx * T::SP, yb = sy * rows, ye = std::min(yb + rows, H);
     const int wk = wv / (TO * TI), wo = wv % (TO * TI) / TI, wi = wv % TI;
 
     f32x4 acc[KS * KS][2][2];
@@ -437,6 +437,7 @@ __global__ void __launch_bounds__(256, 2) wgrad_kernel(const uint16_t *__restric
 #pragma unroll
             for (int b = 0; b < 2; ++b) acc[t][a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+    int n = 0, x0 = 0, ye = 0;   // the strip's image, first column and row end
     u32x4 ri[T::UI], rd[T::UD];
     auto fetch_in = [&](int y) {   // input row y (zeros outside the image)
 #pragma unroll
@@ -472,39 +473,46 @@ __global__ void __launch_bounds__(256, 2) wgrad_kernel(const uint16_t *__restric
             if (px < T::SP) *reinterpret_cast<u32x4 *>(d + px * T::PD + k % (TO * 4) * 8) = rd[u];
         }
     };
-    for (int y = yb - T::R; y <= yb + T::R; ++y) {
-        fetch_in(y);
-        put_in(y);
-    }
-    fetch_dout(yb);
-    put_dout(yb);
     const int fp = 4 * g + i16 / 4, fc = 4 * (i16 % 4);   // a lane's pixel and channel within a fragment
-    for (int y = yb; y < ye; ++y) {
-        __syncthreads();
-        fetch_in(y + T::R + 1);
-        fetch_dout(y + 1);
+    for (int u = int(blockIdx.x); u < strips; u += int(gridDim.x)) {
+        const int yb = u / nsx % nsy * rows;
+        n = u / (nsx * nsy);
+        x0 = u % nsx * T::SP;
+        ye = std::min(yb + rows, H);
+        if (u != int(blockIdx.x)) __syncthreads();   // the rows of the strip before are still read
+        for (int y = yb - T::R; y <= yb + T::R; ++y) {
+            fetch_in(y);
+            put_in(y);
+        }
+        fetch_dout(yb);
+        put_dout(yb);
+        for (int y = yb; y < ye; ++y) {
+            __syncthreads();
+            fetch_in(y + T::R + 1);
+            fetch_dout(y + 1);
 #pragma unroll
-        for (int k = 0; k < T::KPW / 32; ++k) {
-            const int p = wk * T::KPW + 32 * k + fp;
-            bf16x8 A[2];
+            for (int k = 0; k < T::KPW / 32; ++k) {
+                const int p = wk * T::KPW + 32 * k + fp;
+                bf16x8 A[2];
 #pragma unroll
-            for (int a = 0; a < 2; ++a) A[a] = ld_tr(sD(y) + p * T::PD + wo * 32 + 16 * a + fc, T::PD);
+                for (int a = 0; a < 2; ++a) A[a] = ld_tr(sD(y) + p * T::PD + wo * 32 + 16 * a + fc, T::PD);
 #pragma unroll
-            for (int dy = 0; dy < KS; ++dy) {
-                const uint16_t *row = sI(y + dy - T::R) + wi * 32 + fc;
+                for (int dy = 0; dy < KS; ++dy) {
+                    const uint16_t *row = sI(y + dy - T::R) + wi * 32 + fc;
 #pragma unroll
-                for (int dx = 0; dx < KS; ++dx) {
+                    for (int dx = 0; dx < KS; ++dx) {
 #pragma unroll
-                    for (int b = 0; b < 2; ++b) {
-                        const bf16x8 Bv = ld_tr(row + (p + dx) * T::PI + 16 * b, T::PI);
+                        for (int b = 0; b < 2; ++b) {
+                            const bf16x8 Bv = ld_tr(row + (p + dx) * T::PI + 16 * b, T::PI);
 #pragma unroll
-                        for (int a = 0; a < 2; ++a) acc[dy * KS + dx][a][b] = mma(A[a], Bv, acc[dy * KS + dx][a][b]);
+                            for (int a = 0; a < 2; ++a) acc[dy * KS + dx][a][b] = mma(A[a], Bv, acc[dy * KS + dx][a][b]);
+                        }
                     }
                 }
             }
+            put_in(y + T::R + 1);
+            put_dout(y + 1);
         }
-        put_in(y + T::R + 1);
-        put_dout(y + 1);
     }
     // the waves of one channel tile (WK of them) meet in LDS, a tap at a time;
     // each then writes 4 / WK of the tile's four 16 x 16 parts
@@ -911,10 +919,19 @@ void check_view(const void *p, int stride, int channels, const char *what)
 }
 
 // The weight gradient's launch: 64 channels a tile where the count is a multiple
-// of 64, else 32; rows a segment so that at most 512 blocks run (two fit on
-// each of the 256 CUs) where that leaves at least 4.
+// of 64, else 32; rows a segment so that at most kWgradBlocks workgroups run (two
+// fit on each of the 256 CUs) where that leaves at least 4.  Where whole columns
+// of many images are still more strips than that, a workgroup takes several, cut
+// so that all have about as many rows: every workgroup writes a partial tile of
+// all taps, which the reduce pass reads again, so the scratch holds at most
+// kWgradBlocks of them (75 MB at 64 x 64 channels and 3 x 3) or, past 512 channel
+// tiles, one for each.  Measured with one strip a workgroup / as now: 16 x 48 x
+// 144, 256 channels both ways 179 / 166 us (114 / 76 MB), 64 images 735 / 593 (454 / 76),
+// 16 x 24 x 72, 512 channels 276 / 217 (303 / 77).
+constexpr int64_t kWgradBlocks = 512;
+
 struct WgradPlan {
-    int to, ti, nsx, nsy, rows, blocks;
+    int to, ti, nsx, nsy, rows, strips, blocks;
 };
 
 WgradPlan wgrad_plan(int N, int H, int W, int cin, int cout)
@@ -925,10 +942,26 @@ WgradPlan wgrad_plan(int N, int H, int W, int cin, int cout)
     const int wk = 4 / (p.to * p.ti), sp = wk == 4 ? 128 : 64;
     const int64_t tiles = int64_t((cin + 32 * p.ti - 1) / (32 * p.ti)) * ((cout + 32 * p.to - 1) / (32 * p.to));
     p.nsx = (W + sp - 1) / sp;
-    const int64_t want = std::max<int64_t>(1, 512 / (tiles * p.nsx * N));
-    p.rows = int(std::max<int64_t>(std::min(H, 4), (H + want - 1) / want));
+    const int64_t most = std::max<int64_t>(1, kWgradBlocks / tiles);   // workgroups a channel tile
+    const int64_t cols = int64_t(p.nsx) * N;
+    if (cols <= most) {
+        const int64_t want = std::max<int64_t>(1, kWgradBlocks / (tiles * cols));
+        p.rows = int(std::max<int64_t>(std::min(H, 4), (H + want - 1) / want));
+    } else {
+        int64_t best = INT64_MAX;   // rows that the busiest workgroup walks, two more each strip
+        for (int k = 1; k <= 8 && (k == 1 || H / k >= 4); ++k) {
+            const int rows = (H + k - 1) / k;
+            const int64_t cost = (cols * ((H + rows - 1) / rows) + most - 1) / most * (rows + 2);
+            if (cost < best) {
+                best = cost;
+                p.rows = rows;
+            }
+        }
+    }
     p.nsy = (H + p.rows - 1) / p.rows;
-    p.blocks = p.nsx * p.nsy * N;
+    p.strips = p.nsx * p.nsy * N;
+    const int64_t each = (p.strips + most - 1) / most;
+    p.blocks = int((p.strips + each - 1) / each);
     return p;
 }
 
@@ -1005,7 +1038,7 @@ void conv_wgrad(const uint16_t *in, int N, int H, int W, int cin, int in_stride,
                     unsigned((cout + 32 * w.to - 1) / (32 * w.to)));
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream(), in, H, W, cin, in_stride, dout, cout, dout_stride,
-                           partials, w.nsx, w.nsy, w.rows);
+                           partials, w.nsx, w.nsy, w.rows, w.strips);
     };
     const int tile = (w.to - 1) * 2 + w.ti - 1;
     if (ks == 3)

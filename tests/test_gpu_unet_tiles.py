@@ -99,3 +99,11 @@ def test_negative_counts_are_empty():
     _call("swp_nn_up2_fwd", _p(a), C, -1, H, W, C, _p(b), C)
     _call("swp_nn_up2_bwd", _p(b), C, -1, H, W, C, _p(a), C)
     assert torch.equal(a, a0) and torch.equal(b, b0)
+
+
+@pytest.mark.parametrize("N,H,W,cin,cout,ks", [
+    (50, 2, 130, 72, 40, 3), (50, 3, 65, 192, 128, 3), (90, 1, 65, 256, 128, 1), (37, 2, 129, 64, 520, 1)])
+def test_wgrad_several_strips_a_workgroup(N, H, W, cin, cout, ks):
+    """More strips of images than workgroups: each takes several in turn, the
+    last ones perhaps fewer."""
+    test_wgrad_tile_edges(N, H, W, cin, cout, ks)
