@@ -453,6 +453,7 @@ static void launch_recon(const Ctx &x, const float *vp, const float *u_prev, con
         return;
     }
     const dim3 grid = grid_for(bx.x1 - bx.x0, bx.y1 - bx.y0, bx.z1 - bx.z0, g.B);
+    census_add("a3d.recon_cell", int64_t(grid.x) * grid.y * grid.z);
     by_order(g.M, [&](auto ms) {
         hipLaunchKernelGGL(recon_kernel<decltype(ms)::value>, grid, dim3(64, 4), 0, stream(), g, x.c, vp, u_prev,
                            u_now, u_next, adj, grad, bx);

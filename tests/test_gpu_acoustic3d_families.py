@@ -27,8 +27,9 @@ def _memory(name):
 
 
 def _run(order, shape, B, mode, nt=24):
-    """Record, model gradient and launch census of a call whose receivers lie
-    around its sources, so that nt steps carry the wave to them."""
+    """Record, model gradient and launch census of a call with its sources in
+    corners and receivers around them, so that nt steps carry the wave to the
+    receivers, over the strips and into the layers of every axis."""
     from sweep_amd import _core
     from sweep_amd.equations import Acoustic3D
     from sweep_amd.propagator import PropTorch
@@ -40,7 +41,7 @@ def _run(order, shape, B, mode, nt=24):
     t = np.arange(nt) * 1e-3
     a = (np.pi * 40.0 * (t - 0.006)) ** 2
     wav = ((1 - 2 * a) * np.exp(-a)).astype(np.float32)
-    src = np.array([[(nx * (b + 1)) // (B + 1), ny // 2, nz // 2] for b in range(B)])
+    src = np.array([[3, 2, 2], [nx - 4, ny - 3, nz - 3]])[:B]
     off = np.stack(np.meshgrid([-2, 0, 2], [-2, 0, 2], [-1, 0, 1], indexing="ij"), -1).reshape(-1, 3)
     rec = src[:, None, :] + off[None]
     res = rng.standard_normal((B, nt, rec.shape[1], 1)).astype(np.float32)
@@ -90,3 +91,27 @@ def test_default_route(order, shape, B, mode, fwd, adj, monkeypatch):
     print(f"[families] {sorted(sites)} grad {e:.2e}", flush=True)
     assert torch.equal(rec, rec_cell)
     assert e <= 1e-5
+
+
+@pytest.mark.parametrize("order,shape,mode,recon", [
+    (8, (97, 63, 45), "bs", "cell"), (4, (50, 81, 67), "bs", "cell"), (8, (97, 63, 45), "bs_bf16", "cell"),
+    (8, (176, 176, 176), "bs", "zm")])
+def test_default_reconstruction(order, shape, mode, recon, monkeypatch):
+    """Forward and adjoint on the z-march with a reconstruction box on either
+    side of its own border: against full storage (the float32 strips; bar as for
+    the full grids) and against the per-cell kernels."""
+    monkeypatch.delenv("SWP_KERNELS", raising=False)
+    print(f"[families] order={order} shape={shape} {mode}", flush=True)
+    rec, grad, sites = _run(order, shape, 1, mode)
+    assert any(s.startswith("a3d.fwd3.") for s in sites) and any(s.startswith("a3d.adj3.") for s in sites), sites
+    assert {s for s in sites if s.startswith("a3d.recon")} == {f"a3d.recon_{recon}"}
+    if mode == "bs":
+        rec_full, grad_full, _ = _run(order, shape, 1, "full")
+        e = rel_l2(grad, grad_full)
+        print(f"[families] boundary saving against full {e:.2e}", flush=True)
+        assert torch.equal(rec, rec_full)
+        assert e <= 1e-4
+    monkeypatch.setenv("SWP_KERNELS", "percell")
+    rec_cell, grad_cell, _ = _run(order, shape, 1, mode)
+    assert torch.equal(rec, rec_cell)
+    assert rel_l2(grad, grad_cell) <= 1e-5
