@@ -12,10 +12,14 @@ namespace a3d {
 // march_adj in acoustic3d.hip).
 constexpr int64_t kZmMinCells3 = int64_t(4) << 20;
 // From here up the forward step adds the last axes' second derivatives to the
-// CPML sum in one rounding each; below, every term is rounded first, as the
-// per-cell kernels do, so that a record there does not depend on the family.
-// (The records of either range keep the bits they had before the families'
-// border moved down from this size; the times are equal.)
+// CPML sum in one rounding each; below, every term is rounded first, as in the
+// per-cell kernels, so that a record there does not depend on the family.  The
+// times are equal.  It is so for the records' bits: when the border to the
+// per-cell kernels moved down from this size, the records below kept theirs at
+// every order, and those from here up at orders 4, 6 and 8 (order 2's moved, by
+// 7e-7 of the record after 400 steps).  Consequently one shot's record may differ by rounding between
+// launches of few and of many shots.  SWP_KERNELS=zmarch_big runs this form at
+// any size.
 constexpr int64_t kBigCells3 = int64_t(32) << 20;
 // Smallest reconstruction box (shots x cells) on its z-marching kernel: the
 // box holds far fewer cells than the grid, and its kernel walks whole z

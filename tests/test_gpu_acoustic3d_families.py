@@ -115,3 +115,31 @@ def test_default_reconstruction(order, shape, mode, recon, monkeypatch):
     rec_cell, grad_cell, _ = _run(order, shape, 1, mode)
     assert torch.equal(rec, rec_cell)
     assert rel_l2(grad, grad_cell) <= 1e-5
+
+
+@pytest.mark.parametrize("order", [2, 4, 6, 8])
+@pytest.mark.parametrize("mode", ["full", "bs"])
+def test_roundings_of_the_large_sizes_match_oracle(order, mode, monkeypatch):
+    """The forward kernel of 32M shot-cells and up, run on a small grid: every
+    region type, records and gradients against the oracle, and a record that
+    differs from the smaller sizes' by rounding."""
+    import test_gpu_zmarch_interior as zi
+    from sweep_amd.equations import Acoustic3D
+    dev = torch.device("cuda:0")
+    c = zi._case3d(order, seed=80 + order, B=1, nt=100)
+    out = {}
+    for family in ("zmarch", "zmarch_big"):
+        monkeypatch.setenv("SWP_KERNELS", family)
+        out[family] = zi._run(Acoustic3D(spatial_order=order, device=dev), c["shape"], c["dh"], c["dt"], c["abcn"], mode,
+                              c["vp"], c["wav"], c["src"], c["rec"], c["res"], dev)
+    got = out["zmarch_big"]
+    for r in zi.REGIONS:
+        assert got["census"].get(f"a3d.fwd3.{r}", (0, 0))[1] > 0, got["census"]
+    ref = zi._oracle3d(c, mode)
+    errs = {k: rel_l2(got[k], ref[k]) for k in ("rec", "grad_vp", "grad_wavelet")}
+    moved = rel_l2(got["rec"], out["zmarch"]["rec"])
+    print(f"[families] large-size roundings order {order} {mode} {errs}, record moved {moved:.1e}", flush=True)
+    assert errs["rec"] <= 1e-5
+    assert errs["grad_vp"] <= 1e-4
+    assert errs["grad_wavelet"] <= 1e-4
+    assert 0 < moved <= 1e-5

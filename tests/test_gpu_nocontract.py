@@ -185,3 +185,35 @@ def test_elastic2d_random_cases(parity_runs):
                 ref = te._oracle_run(c, st, rt, got.pop("res"), bs=mode == "bs")
                 _compare(f"elastic2d order {order} fields {k} {mode}", got, ref, log)
     _check(log, lambda tag, k: k == "rec" or tag.endswith(" full"))
+
+
+def test_acoustic3d_roundings_of_the_large_sizes(tmp_path):
+    """The forward kernel of 32M shot-cells and up differs from the smaller
+    sizes' only in which products are fused: without contraction its records are
+    the oracle's, bit for bit, too."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import test_gpu_acoustic3d as t3
+    from sweep_amd.build import LIB_NOCONTRACT
+    child = r"""
+import os, sys
+import numpy as np
+sys.path.insert(0, sys.argv[1])
+import test_gpu_acoustic3d as t3
+import torch
+for order in (2, 4, 6, 8):
+    c = t3._random_case(order, seed=order)
+    print(f"[nocontract] acoustic3d order={order} kernels=zmarch_big", flush=True)
+    r = t3._gpu_run(c["order"], c["shape"], c["dh"], c["dt"], c["abcn"], "full", c["vp"], c["wav"], c["src"], c["rec"],
+                    c["res"], torch.device("cuda:0"))
+    np.savez(os.path.join(sys.argv[2], f"big_{order}.npz"), **r)
+"""
+    env = dict(os.environ, SWP_CORE_LIBRARY=str(LIB_NOCONTRACT), PYTHONPATH=str(ROOT), SWP_KERNELS="zmarch_big")
+    r = subprocess.run([sys.executable, "-u", "-c", child, str(TESTS), str(tmp_path)], cwd=ROOT, env=env,
+                       capture_output=True, text=True, timeout=400)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-3000:]
+    log = []
+    for order in (2, 4, 6, 8):
+        ref = t3._oracle_run(t3._random_case(order, seed=order), "full")
+        _compare(f"acoustic3d order {order} zmarch_big full", dict(np.load(tmp_path / f"big_{order}.npz")), ref, log)
+    _check(log, lambda tag, k: k == "rec")
