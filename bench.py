@@ -190,8 +190,8 @@ def elastic_bytes(B, grid, M, pad):
     Forward: velocity {sxx, szz, sxz, rho} -> {vx, vz} (RMW) = 32 B, stress
     {vx, vz, lambda, mu} -> {sxx, szz, sxz} (RMW) = 40 B per computed cell,
     +64 B per band cell (8 memory variables read and written).  Adjoint:
-    stress prepare 36 B, stress apply 32 B, velocity prepare 28 B, velocity
-    apply 40 B per cell, +64 B per band cell.  Imaging: 72 B per physical
+    stress prepare 36 B, stress apply 32 B with the velocity prepare (v from
+    its registers) 20 B, velocity apply 40 B per cell, +64 B per band cell.  Imaging: 72 B per physical
     cell (v(it), v(it+1), the adjoint fields, vp / vs / rho, three gradients
     read and written)."""
     nz, nx = grid
@@ -200,7 +200,7 @@ def elastic_bytes(B, grid, M, pad):
     inner = (nz - 2 * pad - 2 * M) * (nx - 2 * pad - 2 * M)
     band = cells - inner
     phys = inner
-    return {0: B * (72 * cells + 64 * band), 1: B * (36 * allc + 28 * allc + 72 * cells + 64 * (allc - inner)),
+    return {0: B * (72 * cells + 64 * band), 1: B * (36 * allc + 20 * allc + 72 * cells + 64 * (allc - inner)),
             2: B * 72 * phys}
 
 
@@ -269,12 +269,13 @@ REF_SAMPLE_STEPS = {"acoustic3d": 8, "acoustic2d": 1000, "elastic2d": 300, "acou
 # one; any other configuration (another memory mode, shots per launch,
 # --autotune, SWP_TZ* tile overrides) reports None.
 MEASURED_TRAFFIC = {
-    # profiles/acoustic3d_256x512x512_2per_launch_bs.md: the eight region launches of one step
-    ("acoustic3d", "bs", 2): {0: 8.812e9, 1: 10.325e9, 2: 4.770e9},
+    # profiles/acoustic3d_256x512x512_2per_launch_bs.md: forward, adjoint and reconstruction, a launch each
+    ("acoustic3d", "bs", 2): {0: 9.447e9, 1: 11.560e9, 2: 4.657e9},
     # profiles/acoustic2d_384x1152_32shots_bs.md: forward, adjoint (band + interior) and reconstruction
     ("acoustic2d", "bs", 32): {0: 462.7e6, 1: 524.3e6, 2: 433.6e6},
-    # profiles/elastic2d_512x1024_16shots_bs.md: velocity + stress; prepare + apply; imaging
-    ("elastic2d", "bs", 16): {0: 982.9e6, 1: 2677.6e6, 2: 875.9e6},
+    # profiles/elastic2d_512x1024_16shots_bs.md: velocity + stress; stress prepare, apply with the velocity
+    # prepare, velocity apply; imaging
+    ("elastic2d", "bs", 16): {0: 982.8e6, 1: 2554.9e6, 2: 875.4e6},
 }
 TRAFFIC_SOURCE = {
     ("acoustic3d", "bs", 2): "profiles/acoustic3d_256x512x512_2per_launch_bs.md",
