@@ -24,7 +24,7 @@ constexpr int64_t kBigCells3 = int64_t(32) << 20;
 // Smallest reconstruction box (shots x cells) on its z-marching kernel: the
 // box holds far fewer cells than the grid, and its kernel walks whole z
 // segments (1.4M cells 47 us against 16 us per-cell; from 2M to 8M the step
-// times are within 1.5%).
+// times are within 2%).
 constexpr int64_t kZmMinRecon3 = int64_t(4) << 20;
 
 // The cells that the z-march's tiles cover, masked lanes included, over those
